@@ -453,8 +453,16 @@ __device__ __forceinline__ float dec_wave_sum(float v) {
     return v;
 }
 
-template <int DT, int MR, int KS, bool QX>
+// RND: FQ values rounded to the 16-bit operand type before the products, as
+// fused_fake_quantize returns them for such a tensor and the packed path
+// contracts them (axs6_nf5_linear_infer); the fused linear proper keeps them in
+// f32.  The table is staged rounded: rounding commutes with 2^e1 while the
+// value is normal in the type, which bf16 shares with f32; f16 blocks outside
+// e1 in [-6, 15] (lut[0] 2^e1 subnormal, or 2^e1 past its range) take the
+// general sequence and are rounded once more there.
+template <int DT, int MR, int KS, bool QX, bool RND>
 __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) {
+    static_assert(!RND || DT != AXS6_F32, "f32 values need no rounding");
     using E = Elem<DT>;
     using S = typename E::S;
     constexpr int L = dec_loads<DT>();
@@ -510,6 +518,11 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
 #pragma unroll
     for (int u = 0; u < kDecPf; ++u) prefetch(buf[u]);
 
+    if constexpr (RND) {
+        float r[4] = {lutv.x, lutv.y, lutv.z, lutv.w};
+        round_to_elem<DT, 4>(r);
+        lutv = make_float4(r[0], r[1], r[2], r[3]);
+    }
     if (tid < kLutSize / 4) reinterpret_cast<float4*>(lut_s)[tid] = lutv;
     if (tid < kBandSize / 4) band_w[tid] = bandv;
     __syncthreads();
@@ -529,6 +542,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
             const FqScale s = fq_scale(mx, band_s);
             const float d[8] = {};
             fq_vector<8>(f, s, lut_s, false, d);
+            if constexpr (RND) round_to_elem<DT, 8>(f);
         }
         if (c < nchunk) {
             const int m = c / (SP * 64), j = (c / 64) % SP, l = c % 64;
@@ -564,11 +578,13 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
         const int fexp = (int)(mx >> 23) - kExpBias;
         const uint32_t kb = (mx & 0x7f800000u) + 0x00800000u;
         int e1 = (kb - mx <= (uint32_t)band_s[fexp + 150]) ? fexp + 2 : fexp + 1;
-        const bool wide = mx != 0u && (mx < kFastMinAmaxBits || e1 >= 128);
+        bool wide = mx != 0u && (mx < kFastMinAmaxBits || e1 >= 128);
+        if constexpr (RND && DT == AXS6_F16) wide = wide || (mx != 0u && (e1 < -6 || e1 > 15));
         if (__builtin_amdgcn_ballot_w64(wide) != 0) {
             const FqScale s = fq_scale_general(mx, band_s);
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[e] = fq_value(f[e], s, lut_s, false, 0.0f);
+            if constexpr (RND) round_to_elem<DT, 8>(f);
             e1 = 0;
         } else {
             // fq_vector's short sequence without the final 2^e1 (lut_pos: the
@@ -647,13 +663,13 @@ bool decode_form_fits(const FusedK& k) {
     return k.M <= 2 && (int64_t)k.M * sp * kDecStep * (int64_t)sizeof(float) <= kDecXBytes;
 }
 
-template <int DT, int MR, int KS>
+template <int DT, int MR, int KS, bool RND>
 void launch_decode_ks(const FusedK& k, bool qx, hipStream_t st) {
     const int sp = (k.K + kDecStep - 1) / kDecStep;
     const size_t xl = (size_t)MR * sp * kDecStep * sizeof(float);
     const unsigned grid = (unsigned)((k.N + kDecWaves / KS - 1) / (kDecWaves / KS));
-    if (qx) fused_decode_kernel<DT, MR, KS, true><<<grid, kDecWaves * 64, xl, st>>>(k);
-    else fused_decode_kernel<DT, MR, KS, false><<<grid, kDecWaves * 64, xl, st>>>(k);
+    if (qx) fused_decode_kernel<DT, MR, KS, true, RND><<<grid, kDecWaves * 64, xl, st>>>(k);
+    else fused_decode_kernel<DT, MR, KS, false, RND><<<grid, kDecWaves * 64, xl, st>>>(k);
 }
 
 // Two waves per row (each half of the steps) when the rows alone would give
@@ -662,11 +678,17 @@ void launch_decode_ks(const FusedK& k, bool qx, hipStream_t st) {
 // 8192 x 8192 47.4 -> 41.2 us, 8192 x 16000 97.3 -> 87.1 us; one wave per
 // row at 4096 x 4096 12.6 against 13.9 us, 4096 x 32000 89.8 against
 // 106.3 us, 4096 x 128000 324 against 362 us.
-template <int DT, int MR>
+template <int DT, int MR, bool RND>
 void launch_decode(const FusedK& k, bool qx, hipStream_t st) {
     const int sp = (k.K + kDecStep - 1) / kDecStep;
-    if ((sp >= 8 && k.N < 2048) || sp >= 16) launch_decode_ks<DT, MR, 2>(k, qx, st);
-    else launch_decode_ks<DT, MR, 1>(k, qx, st);
+    if ((sp >= 8 && k.N < 2048) || sp >= 16) launch_decode_ks<DT, MR, 2, RND>(k, qx, st);
+    else launch_decode_ks<DT, MR, 1, RND>(k, qx, st);
+}
+
+template <int DT, bool RND>
+void launch_decode_rows(const FusedK& k, bool qx, hipStream_t st) {
+    if (k.M == 1) launch_decode<DT, 1, RND>(k, qx, st);
+    else launch_decode<DT, 2, RND>(k, qx, st);
 }
 
 template <int DT, int WM, int TN, int NW, bool XL = false, bool XA = false>
@@ -729,8 +751,7 @@ void launch_mfma(const FusedK& k, bool qx, hipStream_t st) {
 template <int DT>
 void launch_dt(const FusedK& k, bool qx, hipStream_t st) {
     if (decode_form_fits(k)) {
-        if (k.M == 1) launch_decode<DT, 1>(k, qx, st);
-        else launch_decode<DT, 2>(k, qx, st);
+        launch_decode_rows<DT, false>(k, qx, st);
         return;
     }
     launch_mfma<DT, false>(k, qx, st);
@@ -844,5 +865,44 @@ extern "C" int axs6_nf5_fused_linear_split(const void* x, const void* w, const f
     if (dtype == AXS6_F32) launch_split<AXS6_F32>(k, x_arranged, qx, st);
     else if (dtype == AXS6_BF16) launch_split<AXS6_BF16>(k, x_arranged, qx, st);
     else launch_split<AXS6_F16>(k, x_arranged, qx, st);
+    return check_launch(fn);
+}
+
+// The inference forward: the packed path's results (FQ values in the operands'
+// type) without the packed operands a backward would need.  One or two rows
+// take the streamed decode form: the weight is read once, where the packed path
+// reads it, writes it in fp16 and reads that (1 x 4096 x 11008 f32, three
+// weights in turn, whole call: 69.8 -> 33.3 us, 5.4 TB/s of weight, the rate of
+// a large copy).
+extern "C" int64_t axs6_nf5_linear_infer_workspace(int64_t M, int64_t N, int64_t K, int32_t dtype,
+                                                   int32_t block_size) {
+    if (!valid_dtype(dtype) || block_size != 32 || M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || M > (1 << 30) ||
+        N > (1 << 30) || K > (1 << 30))
+        return -1;
+    const FusedK k{nullptr, nullptr, nullptr, nullptr, (int)M, (int)N, (int)K, nullptr, nullptr};
+    return decode_form_fits(k) ? 0 : -1;
+}
+
+extern "C" int axs6_nf5_linear_infer(const void* x, const void* w, const float* bias, void* y, int32_t dtype,
+                                     int64_t M, int64_t N, int64_t K, int32_t block_size, int32_t quantize_input,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "axs6_nf5_linear_infer";
+    bool empty;
+    int rc = fused_args(fn, x, w, y, dtype, M, N, K, block_size, &empty);
+    if (rc || empty) return rc;
+    const int64_t need = axs6_nf5_linear_infer_workspace(M, N, K, dtype, block_size);
+    if (need < 0) return fail(AXS6_ERR_UNSUPPORTED, "%s: no inference form for this shape (use the forward)", fn);
+    if (need && (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16))
+        return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: workspace of %lld bytes (16-byte aligned) required", fn,
+                    (long long)need);
+    DeviceTables t;
+    rc = device_tables(&t);
+    if (rc) return rc;
+    const FusedK k{x, w, bias, y, (int)M, (int)N, (int)K, t.lut, t.band};
+    hipStream_t st = (hipStream_t)stream;
+    const bool qx = quantize_input != 0;
+    if (dtype == AXS6_F32) launch_decode_rows<AXS6_F32, false>(k, qx, st);
+    else if (dtype == AXS6_BF16) launch_decode_rows<AXS6_BF16, true>(k, qx, st);
+    else launch_decode_rows<AXS6_F16, true>(k, qx, st);
     return check_launch(fn);
 }

@@ -248,8 +248,10 @@ struct Fwd {
     at::ScalarType dtype;
 };
 
+// train = false: no backward will follow, so where the library has an inference
+// form for the shape it runs instead and the packed operands stay undefined.
 Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
-                    int64_t bs, bool quantize_input) {
+                    int64_t bs, bool quantize_input, bool train = true) {
     const char* fn = "axs_linear";
     require_device(input, fn);
     require_device(weight, fn);
@@ -264,6 +266,25 @@ Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std
     const at::ScalarType dtype = compute_dtype(input.scalar_type());
     const int64_t vm = vec_multiple(dtype);
     at::Tensor x2 = dense(pad_last(rows2d(input, K).to(dtype), vm));
+    Fwd r;
+    if (!train) {
+        const int64_t M = x2.size(0);
+        const int64_t ws = axs6_nf5_linear_infer_workspace(M, N, K, dtype_code(dtype), (int32_t)bs);
+        if (ws >= 0) {
+            at::Tensor w2 = dense(weight.to(dtype)), b;
+            if (bias && bias->defined()) b = bias_vector(*bias, N, fn).to(at::kFloat).contiguous();
+            at::Tensor y = at::empty({M, N}, x2.options());
+            at::Tensor work = ws ? at::empty({ws}, x2.options().dtype(at::kByte)) : at::Tensor();
+            c10::DeviceGuard guard(x2.device());
+            check_rc(axs6_nf5_linear_infer(x2.data_ptr(), w2.data_ptr(), b.defined() ? b.data_ptr<float>() : nullptr,
+                                           y.data_ptr(), dtype_code(dtype), M, N, K, (int32_t)bs,
+                                           quantize_input ? 1 : 0, ws ? work.data_ptr() : nullptr, ws,
+                                           stream_of(x2)),
+                     "axs6_nf5_linear_infer");
+            r.out = to_input_dtype(y.reshape(lead_shape(input.sizes(), N)), input.scalar_type());
+            return r;
+        }
+    }
     at::Tensor w2 = dense(pad_rows(pad_last(weight.to(dtype), vm), vm));
     const int64_t M = x2.size(0), Kb = x2.size(1), Nb = w2.size(0);
     at::Tensor b;
@@ -274,7 +295,6 @@ Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std
     }
     const int64_t Kp = axs6_linear_padded_k(Kb);
     const auto dev = x2.options();
-    Fwd r;
     r.xq = at::empty({M, Kp}, dev.dtype(at::kHalf));
     r.wq = at::empty({Nb, Kp}, dev.dtype(at::kHalf));
     r.sx = at::empty({M}, dev.dtype(at::kInt));
@@ -353,9 +373,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> linear_bwd_impl(
 struct LinearFunction : public torch::autograd::Function<LinearFunction> {
     static at::Tensor forward(AutogradContext* ctx, const at::Tensor& input, const at::Tensor& weight,
                               const at::Tensor& bias, int64_t bs, bool quantize_input, bool quantize_grad,
-                              bool has_bias) {
+                              bool has_bias, bool train) {
         Fwd r = linear_fwd_impl(input, weight, has_bias ? std::optional<at::Tensor>(bias) : std::nullopt, bs,
-                                quantize_input);
+                                quantize_input, train);
+        if (!train) return r.out;   // nothing records a gradient: nothing to save
         ctx->save_for_backward({r.xq, r.sx, r.wq, r.sw});
         auto& d = ctx->saved_data;
         d["M"] = r.M; d["N"] = r.N; d["K"] = r.K; d["n_true"] = r.n_true; d["k_true"] = r.k_true;
@@ -372,7 +393,7 @@ struct LinearFunction : public torch::autograd::Function<LinearFunction> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const at::Tensor& g = grads[0];
         if (!g.defined())
-            return {at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+            return variable_list(8);
         const auto saved = ctx->get_saved_variables();
         auto& d = ctx->saved_data;
         const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
@@ -383,7 +404,7 @@ struct LinearFunction : public torch::autograd::Function<LinearFunction> {
             d["n_true"].toInt(), d["k_true"].toInt(), (at::ScalarType)d["dtype"].toInt(), x_shape,
             (at::ScalarType)d["w_dtype"].toInt(), d["bs"].toInt(), d["quantize_grad"].toBool(), need_x, need_w,
             need_b, std::nullopt, (at::ScalarType)d["x_dtype"].toInt());
-        return {dx, dw, db, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+        return {dx, dw, db, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
     }
 };
 
@@ -392,8 +413,11 @@ at::Tensor linear(const at::Tensor& input, const at::Tensor& weight, const std::
     // the autograd node records every tensor argument's device, so a missing
     // bias travels as an empty tensor (no storage) that forward() treats as absent
     const bool has_bias = bias && bias->defined();
+    // what Function::apply tests before it makes the node a backward can reach
+    const bool train = at::GradMode::is_enabled() &&
+                       (input.requires_grad() || weight.requires_grad() || (has_bias && bias->requires_grad()));
     return LinearFunction::apply(input, weight, has_bias ? *bias : at::empty({0}, input.options()), bs,
-                                 quantize_input, quantize_grad, has_bias);
+                                 quantize_input, quantize_grad, has_bias, train);
 }
 
 py::tuple linear_fwd(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,

@@ -1,0 +1,122 @@
+"""The linear without gradients (``axs_linear_unified`` under ``no_grad`` and
+``accelerated_linear``), which takes the library's inference forms where it has
+one for the shape: FQ values in the operands' type, as the training forward.
+
+Bars, rel-L2 against the fp64 product of the oracle's FQ operands rounded to
+the operands' type: the output's rounding, at most its unit roundoff per value
+(2^-9 bf16, 2^-11 f16), on top of the operands' -- none for 16-bit types, whose
+FQ values the 16-bit operands hold exactly, and for f32 the 11-bit rounding of
+both packed operands, 1e-3 (3.2e-4 measured)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+BAR = {torch.float32: 1e-3, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -11}
+
+
+def _inputs(m, K, N, dt, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(m, K, generator=g)
+    x[torch.rand(m, K, generator=g) < 0.01] *= 100.0
+    x[:, 5] = 0.0
+    w = torch.randn(N, K, generator=g) * K ** -0.5
+    w[:, 3] = 0.0
+    return x.to(dt), w.to(dt), torch.randn(N, generator=g).to(dt)
+
+
+def _exact(x, w, b):
+    def q(t):
+        return torch.from_numpy(oracle.fake_quantize(t.float().numpy(), 32)).to(t.dtype).double()
+
+    y = q(x) @ q(w).t()
+    return y if b is None else y + b.double()
+
+
+def _infer(x, w, b):
+    from axs.unified import functional_unified as fu
+
+    with torch.no_grad():
+        return fu.axs_linear_unified(x.to(DEV), w.to(DEV), None if b is None else b.to(DEV))
+
+
+def _form(m, K, N, dt):
+    from axs import _lib
+
+    return _lib.lib().axs6_nf5_linear_infer_workspace(m, N, K, _lib.DTYPE_CODE[dt], 32) >= 0
+
+
+# one and two rows: a row step's edges, K split over two waves (16+ steps, or
+# 8+ with few rows), ragged last steps and row counts
+@pytest.mark.parametrize("dt", list(BAR), ids=str)
+@pytest.mark.parametrize("m,K,N", [(1, 32, 1), (2, 512, 7), (1, 544, 300), (2, 4096, 1030), (1, 8192, 257),
+                                   (2, 4608, 2050)])
+def test_infer_streamed_rows(m, K, N, dt):
+    print(f"[infer {dt} m={m} K={K} N={N}]", flush=True)
+    x, w, b = _inputs(m, K, N, dt, K + N + m)
+    assert _form(m, K, N, dt)
+    y = _infer(x, w, b)
+    assert y.dtype == dt and y.shape == (m, N) and not y.requires_grad
+    assert oracle.rel_l2(y.float().cpu().numpy(), _exact(x, w, b)) <= BAR[dt]
+
+
+@pytest.mark.parametrize("dt", list(BAR), ids=str)
+def test_infer_special_blocks(dt):
+    """NaN, inf, tiny, huge and part-subnormal blocks of the weight."""
+    K, N = 1024, 64
+    x, w, _ = _inputs(2, K, N, dt, 4)
+    big, small, sub = (1e3, 1e-3, 1e-7) if dt == torch.float16 else (1e30, 1e-33, 1e-41)
+    w = w.float()
+    w[3, 100] = float("nan")
+    w[4, 64:96] = w[4, 64:96].abs() + 0.1
+    w[4, 70] = float("inf")
+    w[5] *= small
+    w[6] *= big
+    w[7, 0:32] = sub
+    w[7, 3] = 0.5
+    w = w.to(dt)
+    y = _infer(x, w, None).float().cpu().numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = _exact(x, w, None).numpy()
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
+    for c in (0, 5, 6, 7):       # each row against its own scale
+        assert oracle.rel_l2(y[:, c], want[:, c]) <= 2 * BAR[dt], c
+
+
+def test_infer_keeps_the_training_path_under_grad():
+    """A recorded gradient takes the training forward, bit for bit."""
+    from axs.unified import functional_unified as fu, hip_linear
+
+    x, w, b = (t.to(DEV) for t in _inputs(2, 256, 96, torch.float32, 9))
+    want = hip_linear.forward_train(x, w, b)[0]
+    for needs in ((True, False, False), (False, True, False), (False, False, True)):
+        a = [t.clone().requires_grad_(n) for t, n in zip((x, w, b), needs)]
+        y = fu.axs_linear_unified(*a)
+        assert y.requires_grad and torch.equal(y.detach(), want)
+        y.sum().backward()
+    assert not fu.axs_linear_unified(x, w, b).requires_grad
+
+
+def test_infer_in_graph_replays():
+    x, w, b = (t.to(DEV) for t in _inputs(1, 4096, 1030, torch.bfloat16, 11))
+    eager = _infer(x, w, b)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _infer(x, w, b)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = _infer(x, w, b)
+    for i in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager), i
