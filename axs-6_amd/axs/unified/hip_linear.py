@@ -168,14 +168,18 @@ def fused_forward(input, weight, bias=None, quantize_input=True):
 def linear_forward(input, weight, bias=None, block_size=32, quantize_input=True):
     """Y = FQ(input) FQ(weight)^T + bias (no autograd bookkeeping): the fused
     single-launch kernel for block size 32 and at most FUSED_SIZE_THRESHOLD
-    outputs, else the packing kernels and the fp16-MFMA GEMM.  Y has the
-    input's dtype."""
+    outputs, else the extension's forward without gradients (axs._C.linear_infer:
+    the library's inference form where it has one for the shape, else the packing
+    kernels and the fp16-MFMA GEMM).  Y has the input's dtype."""
     if block_size == 32 and input.shape[-1] == weight.shape[-1]:
         rows = input.numel() // input.shape[-1] if input.shape[-1] else 0
         if rows * weight.shape[0] <= FUSED_SIZE_THRESHOLD:
             return fused_forward(input, weight, bias, quantize_input)
-    out, _ = _forward(input, weight, bias, block_size, quantize_input)
-    return out
+    fn = "axs_linear"
+    _require_device(input, fn)
+    _require_device(weight, fn)
+    assert block_size in VALID_BLOCK_SIZES, f"block_size must be one of {VALID_BLOCK_SIZES}"
+    return _lib.ext().linear_infer(input, weight, bias, block_size, bool(quantize_input))
 
 
 def backward(grad_output, saved: Saved, block_size: int, quantize_grad: bool,

@@ -129,6 +129,11 @@ bool gemm_pairs(const GemmArgs& a, const GemmArgs& b);
 int gemm_split_count(int64_t M, int64_t N, int64_t Kp);
 size_t gemm_split_bytes(int64_t M, int64_t N, int64_t Kp);
 
+// The streamed form of the linear without gradients (nf5_fused_linear.hip).
+bool infer_rows_fit(int64_t M, int64_t N, int64_t K);
+int launch_infer_rows(const void* x, const void* w, const void* bias, int bias_dtype, void* y, int dtype, int64_t M,
+                      int64_t N, int64_t K, bool qx, const DeviceTables& t, hipStream_t st);
+
 constexpr int64_t kGemmK = 64;   // contraction padding unit
 inline int64_t pad_to(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 

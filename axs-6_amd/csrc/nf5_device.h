@@ -110,6 +110,13 @@ template <> struct Elem<AXS6_F16> {
     }
 };
 
+// Element i of an array whose type is known at run time (a bias).
+__device__ __forceinline__ float load_elem(const void* p, int dtype, int64_t i) {
+    if (dtype == AXS6_F32) return reinterpret_cast<const float*>(p)[i];
+    if (dtype == AXS6_BF16) return Elem<AXS6_BF16>::to_f(reinterpret_cast<const uint16_t*>(p)[i]);
+    return Elem<AXS6_F16>::to_f(reinterpret_cast<const _Float16*>(p)[i]);
+}
+
 // ---- block arithmetic ------------------------------------------------------
 
 // v and the value DPP control `ctrl` brings to this lane, unsigned max.  Every

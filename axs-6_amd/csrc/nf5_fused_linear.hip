@@ -44,6 +44,8 @@
 // back to the input dtype).
 #include "nf5_device.h"
 
+#include "linear_internal.h"
+
 namespace axs6 {
 namespace {
 
@@ -58,9 +60,10 @@ constexpr int kFRed = 32 * 1024;     // bytes of LDS for the partial tiles
 constexpr int kXlBytes = 139 * 1024;
 
 struct FusedK {
-    const void* x; const void* w; const float* bias; void* y;
+    const void* x; const void* w; const void* bias; void* y;
     int M; int N; int K;
     const float* lut; const uint8_t* band;
+    int bias_dtype = AXS6_F32;
 };
 
 // The 8 values lane (row r, group q) takes of a row's 32-block: in bf16/f16
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(NW * 64) void fused_linear_kernel(FusedK k) {
         float v = red[o];
 #pragma unroll
         for (int w = 1; w < NW; ++w) v += red[w * (BM * BN) + o];
-        if (k.bias) v += k.bias[n];
+        if (k.bias) v += load_elem(k.bias, k.bias_dtype, n);
         reinterpret_cast<S*>(k.y)[(int64_t)m * k.N + n] = E::from_f(v);
     }
 }
@@ -650,7 +653,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
         }
     }
     if (ks == 0 && lane == 0 && live) {
-        const float bn = k.bias ? k.bias[n] : 0.0f;
+        const float bn = k.bias ? load_elem(k.bias, k.bias_dtype, n) : 0.0f;
 #pragma unroll
         for (int m = 0; m < MR; ++m)
             if (m < k.M) reinterpret_cast<S*>(k.y)[(int64_t)m * k.N + n] = E::from_f(t[m] + bn);
@@ -868,41 +871,25 @@ extern "C" int axs6_nf5_fused_linear_split(const void* x, const void* w, const f
     return check_launch(fn);
 }
 
-// The inference forward: the packed path's results (FQ values in the operands'
-// type) without the packed operands a backward would need.  One or two rows
-// take the streamed decode form: the weight is read once, where the packed path
-// reads it, writes it in fp16 and reads that (1 x 4096 x 11008 f32, three
-// weights in turn, whole call: 69.8 -> 33.3 us, 5.4 TB/s of weight, the rate of
-// a large copy).
-extern "C" int64_t axs6_nf5_linear_infer_workspace(int64_t M, int64_t N, int64_t K, int32_t dtype,
-                                                   int32_t block_size) {
-    if (!valid_dtype(dtype) || block_size != 32 || M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || M > (1 << 30) ||
-        N > (1 << 30) || K > (1 << 30))
-        return -1;
-    const FusedK k{nullptr, nullptr, nullptr, nullptr, (int)M, (int)N, (int)K, nullptr, nullptr};
-    return decode_form_fits(k) ? 0 : -1;
+// The inference forward at one or two rows (axs6_nf5_linear_infer): the packed
+// path's results, FQ values in the operands' type, from the streamed form.  The
+// weight is read once, where the packed path reads it, writes it in fp16 and
+// reads that (1 x 4096 x 11008 f32, three weights in turn, whole call: 69.8 ->
+// 33.3 us, 5.4 TB/s of weight, the rate of a large copy).
+namespace axs6 {
+
+bool infer_rows_fit(int64_t M, int64_t N, int64_t K) {
+    return M <= 2 && decode_form_fits(FusedK{nullptr, nullptr, nullptr, nullptr, (int)M, (int)N, (int)K, nullptr,
+                                             nullptr});
 }
 
-extern "C" int axs6_nf5_linear_infer(const void* x, const void* w, const float* bias, void* y, int32_t dtype,
-                                     int64_t M, int64_t N, int64_t K, int32_t block_size, int32_t quantize_input,
-                                     void* workspace, int64_t workspace_bytes, void* stream) {
-    const char* fn = "axs6_nf5_linear_infer";
-    bool empty;
-    int rc = fused_args(fn, x, w, y, dtype, M, N, K, block_size, &empty);
-    if (rc || empty) return rc;
-    const int64_t need = axs6_nf5_linear_infer_workspace(M, N, K, dtype, block_size);
-    if (need < 0) return fail(AXS6_ERR_UNSUPPORTED, "%s: no inference form for this shape (use the forward)", fn);
-    if (need && (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16))
-        return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: workspace of %lld bytes (16-byte aligned) required", fn,
-                    (long long)need);
-    DeviceTables t;
-    rc = device_tables(&t);
-    if (rc) return rc;
-    const FusedK k{x, w, bias, y, (int)M, (int)N, (int)K, t.lut, t.band};
-    hipStream_t st = (hipStream_t)stream;
-    const bool qx = quantize_input != 0;
+int launch_infer_rows(const void* x, const void* w, const void* bias, int bias_dtype, void* y, int dtype, int64_t M,
+                      int64_t N, int64_t K, bool qx, const DeviceTables& t, hipStream_t st) {
+    const FusedK k{x, w, bias, y, (int)M, (int)N, (int)K, t.lut, t.band, bias_dtype};
     if (dtype == AXS6_F32) launch_decode_rows<AXS6_F32, false>(k, qx, st);
     else if (dtype == AXS6_BF16) launch_decode_rows<AXS6_BF16, true>(k, qx, st);
     else launch_decode_rows<AXS6_F16, true>(k, qx, st);
-    return check_launch(fn);
+    return check_launch("infer_rows");
 }
+
+}  // namespace axs6

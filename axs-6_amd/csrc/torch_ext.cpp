@@ -272,14 +272,17 @@ Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std
         const int64_t ws = axs6_nf5_linear_infer_workspace(M, N, K, dtype_code(dtype), (int32_t)bs);
         if (ws >= 0) {
             at::Tensor w2 = dense(weight.to(dtype)), b;
-            if (bias && bias->defined()) b = bias_vector(*bias, N, fn).to(at::kFloat).contiguous();
+            if (bias && bias->defined()) {
+                b = bias_vector(*bias, N, fn);
+                b = (dtype_code(b.scalar_type()) >= 0 ? b : b.to(at::kFloat)).contiguous();
+            }
             at::Tensor y = at::empty({M, N}, x2.options());
             at::Tensor work = ws ? at::empty({ws}, x2.options().dtype(at::kByte)) : at::Tensor();
             c10::DeviceGuard guard(x2.device());
-            check_rc(axs6_nf5_linear_infer(x2.data_ptr(), w2.data_ptr(), b.defined() ? b.data_ptr<float>() : nullptr,
-                                           y.data_ptr(), dtype_code(dtype), M, N, K, (int32_t)bs,
-                                           quantize_input ? 1 : 0, ws ? work.data_ptr() : nullptr, ws,
-                                           stream_of(x2)),
+            check_rc(axs6_nf5_linear_infer(x2.data_ptr(), w2.data_ptr(), b.defined() ? b.data_ptr() : nullptr,
+                                           b.defined() ? dtype_code(b.scalar_type()) : AXS6_F32, y.data_ptr(),
+                                           dtype_code(dtype), M, N, K, (int32_t)bs, quantize_input ? 1 : 0,
+                                           ws ? work.data_ptr() : nullptr, ws, stream_of(x2)),
                      "axs6_nf5_linear_infer");
             r.out = to_input_dtype(y.reshape(lead_shape(input.sizes(), N)), input.scalar_type());
             return r;
@@ -420,6 +423,12 @@ at::Tensor linear(const at::Tensor& input, const at::Tensor& weight, const std::
                                  quantize_input, quantize_grad, has_bias, train);
 }
 
+// The forward alone, no gradient recorded.
+at::Tensor linear_infer(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
+                        int64_t bs, bool quantize_input) {
+    return linear_fwd_impl(input, weight, bias, bs, quantize_input, false).out;
+}
+
 py::tuple linear_fwd(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
                      int64_t bs, bool quantize_input) {
     Fwd r = linear_fwd_impl(input, weight, bias, bs, quantize_input);
@@ -524,6 +533,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("linear", &linear, "FQ(input) FQ(weight)^T + bias with the quantized backward (autograd node)",
           py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("block_size"), py::arg("quantize_input"),
           py::arg("quantize_grad"));
+    m.def("linear_infer", &linear_infer, "the forward alone: FQ(input) FQ(weight)^T + bias (no autograd)",
+          py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("block_size"), py::arg("quantize_input"));
     m.def("linear_fwd", &linear_fwd,
           "forward: (out, xq, sx, wq, sw, M, N, K, n_true, k_true, dtype) -- packed operands for the backward",
           py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("block_size"), py::arg("quantize_input"));

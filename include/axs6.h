@@ -272,7 +272,8 @@ int axs6_nf5_fused_linear_split(const void* x, const void* w, const float* bias,
  * operands' type, as axs6_nf5_linear_forward computes it (equal to its
  * operand rounding), but with no packed operands left for a backward, for the
  * shapes where that is faster.  x [M, K], w [N, K] dense and 16-byte aligned,
- * K a multiple of 32, block_size 32.  axs6_nf5_linear_infer_workspace is a
+ * K a multiple of 32, block_size 32; bias may be null, else N values of
+ * bias_dtype.  axs6_nf5_linear_infer_workspace is a
  * host-only query: the bytes of workspace the call takes (overwritten, 16-byte
  * aligned; may be 0), or -1 where there is no such form and the caller uses
  * axs6_nf5_linear_forward (axs6_nf5_linear_infer then returns
@@ -281,9 +282,9 @@ int axs6_nf5_fused_linear_split(const void* x, const void* w, const float* bias,
  * functional_unified.py:107-131) where no gradient is recorded, and
  * accelerated_linear (axs/unified/backend.py:540) above 128K outputs. */
 int64_t axs6_nf5_linear_infer_workspace(int64_t M, int64_t N, int64_t K, int32_t dtype, int32_t block_size);
-int axs6_nf5_linear_infer(const void* x, const void* w, const float* bias, void* y, int32_t dtype,
-                          int64_t M, int64_t N, int64_t K, int32_t block_size, int32_t quantize_input,
-                          void* workspace, int64_t workspace_bytes, void* stream);
+int axs6_nf5_linear_infer(const void* x, const void* w, const void* bias, int32_t bias_dtype, void* y,
+                          int32_t dtype, int64_t M, int64_t N, int64_t K, int32_t block_size,
+                          int32_t quantize_input, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Device workspace (bytes) axs6_nf5_linear_backward needs for the requested
  * gradients. */

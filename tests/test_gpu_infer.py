@@ -66,11 +66,42 @@ def test_infer_streamed_rows(m, K, N, dt):
     assert oracle.rel_l2(y.float().cpu().numpy(), _exact(x, w, b)) <= BAR[dt]
 
 
+# the weight quantized inside the GEMM: every row tile (32, 64, 128, 256) at its
+# edges, ragged column tiles, N off the 4-value store, K ending in half a step,
+# K split over workgroups and (the last) not
 @pytest.mark.parametrize("dt", list(BAR), ids=str)
-def test_infer_special_blocks(dt):
+@pytest.mark.parametrize("m,K,N", [(3, 1056, 4030), (32, 4096, 1024), (33, 2080, 2051), (64, 1024, 4224),
+                                   (65, 4128, 2049), (128, 8192, 1027), (129, 2048, 4096), (256, 3104, 2710),
+                                   (5, 1024, 65540)])
+def test_infer_gemm(m, K, N, dt):
+    print(f"[infer gemm {dt} m={m} K={K} N={N}]", flush=True)
+    x, w, b = _inputs(m, K, N, dt, K + N + m)
+    assert _form(m, K, N, dt) or (dt == torch.float32 and m > 128)
+    y = _infer(x, w, b)
+    assert y.dtype == dt and y.shape == (m, N)
+    assert oracle.rel_l2(y.float().cpu().numpy(), _exact(x, w, b)) <= BAR[dt]
+    assert torch.equal(_infer(x, w, b), y)     # fixed summation order
+
+
+@pytest.mark.parametrize("dt", list(BAR), ids=str)
+def test_infer_gemm_raw_input(dt):
+    from axs.unified import functional_unified as fu
+
+    x, w, _ = _inputs(48, 1024, 4096, dt, 2)
+    assert _form(48, 1024, 4096, dt)
+    with torch.no_grad():
+        y = fu.axs_linear_unified(x.to(DEV), w.to(DEV), None, 32, False)
+    wq = torch.from_numpy(oracle.fake_quantize(w.float().numpy(), 32)).to(dt).double()
+    assert oracle.rel_l2(y.float().cpu().numpy(), x.double() @ wq.t()) <= BAR[dt]
+
+
+@pytest.mark.parametrize("dt", list(BAR), ids=str)
+@pytest.mark.parametrize("m,N", [(2, 64), (20, 4160), (100, 8200)])
+def test_infer_special_blocks(m, N, dt):
     """NaN, inf, tiny, huge and part-subnormal blocks of the weight."""
-    K, N = 1024, 64
-    x, w, _ = _inputs(2, K, N, dt, 4)
+    K = 1024
+    assert _form(m, K, N, dt)
+    x, w, _ = _inputs(m, K, N, dt, 4)
     big, small, sub = (1e3, 1e-3, 1e-7) if dt == torch.float16 else (1e30, 1e-33, 1e-41)
     w = w.float()
     w[3, 100] = float("nan")
@@ -103,8 +134,9 @@ def test_infer_keeps_the_training_path_under_grad():
     assert not fu.axs_linear_unified(x, w, b).requires_grad
 
 
-def test_infer_in_graph_replays():
-    x, w, b = (t.to(DEV) for t in _inputs(1, 4096, 1030, torch.bfloat16, 11))
+@pytest.mark.parametrize("m", [1, 40])
+def test_infer_in_graph_replays(m):
+    x, w, b = (t.to(DEV) for t in _inputs(m, 4096, 1030, torch.bfloat16, 11))
     eager = _infer(x, w, b)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
