@@ -21,11 +21,10 @@
 // LUT and the band table are staged in LDS once per workgroup and the grid
 // is capped (grid-stride loop) so that staging is amortised.
 // Row path (rows of >= 64 values with a ragged last block, or unaligned
-// views): four values (or one) per lane in row order, a block is
-// `block` / 4 (or `block`) neighbouring lanes (DPP / permlane maximum), rows
-// cut into segments of 256 (or 64) values, the next segment's loads in
-// flight (fq_rows_kernel).  Shorter rows: whole rows per wave, one value per
-// lane, block maxima by segmented shuffle reductions (fq_short_kernel).
+// views): the same 16 bytes per lane, by unaligned accesses, each row padded
+// to whole blocks of lanes (fq_rows_kernel).  Shorter rows: whole rows per
+// wave, one value per lane (four where the rows are whole aligned groups of
+// four), block maxima by segmented shuffle reductions (fq_short_kernel).
 #include <math.h>
 
 #include <type_traits>
@@ -218,107 +217,121 @@ __global__ __launch_bounds__(kThreads) void fq_short_kernel(const typename Elem<
     }
 }
 
+// 16 bytes at any element's address: one unaligned load or store (a wave's 64
+// of them still cover one contiguous KiB, over nine lines instead of eight).
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
+template <int DT> using UnalignedVec = typename std::conditional<DT == AXS6_F32, u32x4_at4, u32x4_at2>::type;
+
 // Rows that do not tile into 16-byte vectors of whole blocks (a ragged last
-// block, or row starts off 16-byte alignment): VL values per lane (4 when
-// the row length is a multiple of 4 and the pointers allow 4-value loads,
-// else 1), lanes in row order, so a block is BS / VL neighbouring lanes and
-// its maximum a DPP (and, for 32 lanes, permlane) reduction; a load or store
-// instruction covers 64 * VL consecutive values of one row.  A row is cut
-// into segments of 64 * VL * U values (a multiple of BS, so blocks never
-// straddle segments); each wave walks a contiguous range of segments,
-// stepping its row index instead of dividing, with the next segment's loads
-// in flight.  Lanes past the row's end read 0 -- the reference's zero
-// padding of the last block -- and store nothing.
-template <int DT, int BS, bool STOCH, int U, int VL>
+// block, or rows off 16-byte alignment), of kRowsMinCols or more values.  A row
+// is gp groups of V values (16 bytes), its last block's padding included, so a
+// block is BS / V neighbouring lanes of one wave whatever the row; lanes take
+// the tensor's groups in order, a thread kRowsUnroll of them, 256 apart, from
+// one division of the workgroup's first group and steps after it.  A group
+// that the row's end cuts loads the row's last V values and shifts them down
+// (zeros above: the reference's padding of the last block) and stores value
+// by value; groups past it hold zeros and store nothing.
+//
+// What bounds it: VALU work per group, as in the vector kernel, and its bytes.
+// The kernel before it took one value per lane wherever a row's length or
+// start was no multiple of 4 values, and so the block's maximum, scale and
+// addresses once per value; four per lane elsewhere.  us, three inputs and
+// outputs in turn, before -> now (nearest; stochastic):
+//   8192 x 4095 bf16   57.0 -> 25.5   70.9 -> 39.8
+//   8192 x 4095 f32    57.9 -> 49.3   62.2 -> 50.6
+//   32768 x 1000 bf16  31.3 -> 25.9   38.5 -> 35.9
+//   2000 x 11007 bf16  35.3 -> 16.6   42.8 -> 23.5
+//   65536 x 300 f32    36.2 -> 27.2   39.2 -> 30.4
+// Three groups a thread (2, 4 and 6: up to 8% longer); streaming stores (plain
+// ones 31.9 and 45.4 us in the first line), plain loads (streaming ones 29.0
+// and 41.1: neighbouring waves share a line).
+constexpr int kRowsUnroll = 3;
+
+template <int DT, int BS, bool STOCH>
 __global__ __launch_bounds__(kThreads) void fq_rows_kernel(const typename Elem<DT>::S* __restrict__ x,
-                                                           typename Elem<DT>::S* __restrict__ y, int64_t rows,
-                                                           int64_t cols, int64_t segs_per_row, int64_t segs_per_wave,
-                                                           const float* __restrict__ lut_g,
+                                                           typename Elem<DT>::S* __restrict__ y, int64_t groups,
+                                                           int64_t cols, int64_t gp, const float* __restrict__ lut_g,
                                                            const uint8_t* __restrict__ band_g, uint64_t seed,
                                                            const uint64_t* __restrict__ seed_dev, uint64_t offset) {
     using E = Elem<DT>;
-    constexpr int SEG = 64 * VL * U;
-    static_assert(VL == 1 || VL == 4, "values per lane");
-    static_assert(SEG % BS == 0 && BS % VL == 0, "segments hold whole blocks");
+    constexpr int V = E::V;
+    static_assert(BS % V == 0, "a group lies inside one block");
     const uint64_t key = STOCH ? dither_key(seed + (seed_dev ? *seed_dev : 0ull)) : 0ull;
     __shared__ float lut_s[kLutSize];
     __shared__ uint32_t band_w[kBandSize / 4];
-    stage_tables(lut_s, band_w, lut_g, band_g);
     const uint8_t* band_s = reinterpret_cast<const uint8_t*>(band_w);
-
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t total = rows * segs_per_row;
-    int64_t seg = wave * segs_per_wave;
-    const int64_t end = seg + segs_per_wave < total ? seg + segs_per_wave : total;
-    if (seg >= end) return;
-    int64_t r = seg / segs_per_row;
-    int64_t sx = seg - r * segs_per_row;
-    // raw words of segment (row rr, index ss) for this lane, zero past the
-    // row's end; converted to floats only when the segment is processed, so
-    // the loads of the next segment stay in flight meanwhile
-    using Raw = typename std::conditional<VL == 1, typename E::S, u32x4>::type;
-    auto load_seg = [&](int64_t rr, int64_t ss, Raw (&w)[U]) {
+    const int tid = threadIdx.x;
+    const int64_t l0 = (int64_t)blockIdx.x * (kThreads * kRowsUnroll);
+    int64_t row[kRowsUnroll], col[kRowsUnroll];
+    u32x4 raw[kRowsUnroll];
+    {
+        const int64_t r0 = l0 / gp;                    // uniform
+        int64_t r = r0, g = l0 - r0 * gp + tid;
+        if (gp <= kThreads) {                          // 32-bit: g < gp + 256
+            const uint32_t q = (uint32_t)g / (uint32_t)gp;
+            r += q;
+            g -= (int64_t)q * gp;
+        } else if (g >= gp) {
+            ++r;
+            g -= gp;
+        }
+        const int64_t dr = kThreads / gp, dg = kThreads - dr * gp;
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const int64_t c = ss * SEG + VL * lane + 64 * VL * k;
-            if constexpr (VL == 1) {
-                w[k] = c < cols ? x[rr * cols + c] : (typename E::S)0;
-            } else if constexpr (DT == AXS6_F32) {
-                w[k] = c < cols ? *reinterpret_cast<const u32x4*>(x + rr * cols + c) : u32x4{0u, 0u, 0u, 0u};
-            } else {
-                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-                const u32x2 h = c < cols ? *reinterpret_cast<const u32x2*>(x + rr * cols + c) : u32x2{0u, 0u};
-                w[k] = u32x4{h.x, h.y, 0u, 0u};
+        for (int u = 0; u < kRowsUnroll; ++u) {
+            const bool live = l0 + u * kThreads + tid < groups;
+            row[u] = live ? r : 0;
+            col[u] = live ? g * V : cols;              // past the row: zeros, nothing stored
+            // inside the row whatever the group (cols >= V)
+            const int64_t c = col[u] + V <= cols ? col[u] : cols - V;
+            raw[u] = *reinterpret_cast<const UnalignedVec<DT>*>(x + row[u] * cols + c);
+            r += dr;
+            g += dg;
+            if (g >= gp) {
+                ++r;
+                g -= gp;
             }
         }
-    };
-    Raw nw[U];
-    load_seg(r, sx, nw);
-    for (; seg < end; ++seg) {
-        const int64_t base = r * cols;
-        float f[U][VL];
+    }
+    stage_tables(lut_s, band_w, lut_g, band_g);
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            if constexpr (VL == 1) {
-                f[k][0] = E::to_f(nw[k]);
-            } else {
-                float g[E::V];
-                E::unpack(nw[k], g);
+    for (int u = 0; u < kRowsUnroll; ++u) {
+        const int64_t base = row[u] * cols + col[u];
+        float f[V];
+        E::unpack(raw[u], f);
+        const bool cut = col[u] + V > cols;
+        if (__builtin_amdgcn_ballot_w64(cut) != 0) {   // wave-uniform: a row ends in this wave
+            const int keep = (int)(cols - col[u] > 0 ? cols - col[u] : 0);   // values of a cut group
+            float g[V];
 #pragma unroll
-                for (int e = 0; e < VL; ++e) f[k][e] = g[e];
+            for (int e = 0; e < V; ++e) {
+                g[e] = 0.0f;
+                // value e is loaded value V - keep + e
+#pragma unroll
+                for (int k = e + 1; k < V; ++k) g[e] = keep == V - (k - e) && k < V ? f[k] : g[e];
             }
-        }
-        int64_t rn = r, sn = sx + 1;
-        if (sn == segs_per_row) {
-            sn = 0;
-            ++rn;
-        }
-        if (seg + 1 < end) load_seg(rn, sn, nw);
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const int64_t c = sx * SEG + VL * lane + 64 * VL * k;
-            uint32_t a = 0;
-#pragma unroll
-            for (int e = 0; e < VL; ++e) {
-                const uint32_t b = __float_as_uint(f[k][e]) & 0x7fffffffu;
-                a = a > b ? a : b;
-            }
-            uint32_t m;
-            if constexpr (VL == 1) m = lanes_umax<BS>(a);
-            else m = group_umax<BS / VL>(a);
-            const FqScale s = fq_scale(m, band_s);
-            float d[VL];
-#pragma unroll
-            for (int e = 0; e < VL; ++e) d[e] = STOCH ? dither_step(key, offset + (uint64_t)(base + c + e)) : 0.0f;
-            fq_vector<VL>(f[k], s, lut_s, STOCH, d);
-            if (c < cols) {
-                if constexpr (VL == 1) y[base + c] = E::from_f(f[k][0]);
-                else store4<DT>(y + base + c, f[k]);
-            }
+            for (int e = 0; e < V; ++e) f[e] = cut ? g[e] : f[e];
         }
-        r = rn;
-        sx = sn;
+        uint32_t m = 0;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const uint32_t a = __float_as_uint(f[e]) & 0x7fffffffu;
+            m = m > a ? m : a;
+        }
+        const FqScale s = fq_scale(group_umax<BS / V>(m), band_s);
+        float d[V];
+        const DitherVec dv = dither_vec(key, offset + (uint64_t)base);
+#pragma unroll
+        for (int e = 0; e < V; ++e) d[e] = STOCH ? dither_step(dv, e) : 0.0f;
+        fq_vector<V>(f, s, lut_s, STOCH, d);
+        if (!cut) {
+            st_stream((UnalignedVec<DT>)E::pack(f), reinterpret_cast<UnalignedVec<DT>*>(y + base));
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                if (col[u] + e < cols) y[base + e] = E::from_f(f[e]);
+        }
     }
 }
 
@@ -624,10 +637,13 @@ __global__ __launch_bounds__(kThreads) void dequantize_kernel(const uint8_t* __r
 }
 
 // Row-segment forms of quantize_kernel and dequantize_kernel, for rows of at
-// least 64 values that do not tile into vectors of whole blocks: the lane
-// and segment layout of fq_rows_kernel over the padded row (cpad = nblk * BS
-// values: the codes and signs of the padding positions are written too, as
-// quantize_kernel writes them), one value per lane.
+// least 64 values that do not tile into vectors of whole blocks: VL values per
+// lane (4 where the row length and pointers allow 4-value loads, else 1), lanes
+// in row order over the padded row (cpad = nblk * BS values: the codes and
+// signs of the padding positions are written too, as quantize_kernel writes
+// them), so a block is BS / VL neighbouring lanes.  A row is cut into segments
+// of 64 * VL * U values; a wave walks a contiguous range of them with the next
+// segment's loads in flight.
 template <int DT, int BS, bool STOCH, int U, int VL>
 __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(
     const typename Elem<DT>::S* __restrict__ x, int64_t rows, int64_t cols, int64_t nblk, int64_t segs_per_row,
@@ -856,7 +872,7 @@ int64_t capped_grid(int64_t work_items, int64_t per_wg) {
     return need < cap ? need : cap;
 }
 
-// Row-segment launches (fq_rows_kernel and its quantize counterpart) for rows
+// Row-segment launches (the quantize and dequantize of ragged rows) for rows
 // of at least kRowsMinCols elements; shorter rows take the short-row kernels
 // (whole rows per wave step).  Segments of 64 * u elements, a contiguous range of per_wave of
 // them per wave, sized for about kRowsWavesPerCu waves per CU and at least
@@ -906,20 +922,14 @@ void launch_fq_typed(const void* x, void* y, int64_t rows, int64_t cols, bool st
     const int esize = (int)sizeof(S);
     const bool four = cols % 4 == 0 && (uintptr_t)x % (4 * esize) == 0 && (uintptr_t)y % (4 * esize) == 0;
     if (cols >= 4 * kRowsMinCols || (cols >= kRowsMinCols && !four)) {
-#define AXS6_FQROWS(U_, VL_)                                                                                   \
-        do {                                                                                                   \
-            const RowSegs g = row_segs(rows, cols, (U_) * (VL_));                                              \
-            if (stochastic)                                                                                    \
-                fq_rows_kernel<DT, BS, true, U_, VL_><<<g.grid, kThreads, 0, st>>>(                            \
-                    (const S*)x, (S*)y, rows, cols, g.per_row, g.per_wave, t.lut, t.band, seed, seed_dev, offset); \
-            else                                                                                               \
-                fq_rows_kernel<DT, BS, false, U_, VL_><<<g.grid, kThreads, 0, st>>>(                           \
-                    (const S*)x, (S*)y, rows, cols, g.per_row, g.per_wave, t.lut, t.band, seed, seed_dev, offset); \
-        } while (0)
-        if (four) AXS6_FQROWS(1, 4);
-        else if (cols >= 4 * kRowsMinCols) AXS6_FQROWS(4, 1);
-        else AXS6_FQROWS(1, 1);
-#undef AXS6_FQROWS
+        const int64_t gp = (cols + BS - 1) / BS * (BS / V), groups = rows * gp;
+        const dim3 grid((unsigned)((groups + kThreads * kRowsUnroll - 1) / (kThreads * kRowsUnroll)));
+        if (stochastic)
+            fq_rows_kernel<DT, BS, true><<<grid, kThreads, 0, st>>>((const S*)x, (S*)y, groups, cols, gp, t.lut, t.band, seed,
+                                                                    seed_dev, offset);
+        else
+            fq_rows_kernel<DT, BS, false><<<grid, kThreads, 0, st>>>((const S*)x, (S*)y, groups, cols, gp, t.lut, t.band,
+                                                                     seed, seed_dev, offset);
     } else {
         // short rows: 1..63 values one per lane, or whole 4-value groups under
         // 256 values (aligned) four per lane; R = 64 * VL / cols rows per wave

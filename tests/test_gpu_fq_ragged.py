@@ -1,0 +1,49 @@
+"""Fake-quantize of rows that do not tile into 16-byte vectors of whole blocks
+(``fq_rows_kernel``: unaligned 16-byte groups, rows padded to whole blocks of
+lanes), bit for bit against the oracle: every length of a cut group, rows of
+fewer and more groups than a workgroup steps by (256), rows shorter and longer
+than a workgroup's share, and a tensor whose last group is its last bytes."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+SEED = 11
+
+# cut groups of 1 .. 7 values; 1017 and 1033: 128 (f32: 256) groups and one more
+# block; 2041 and 2049: 256 (f32: 512) and more; 9001: several workgroups a row
+COLS = [65, 66, 67, 68, 69, 70, 71, 127, 257, 1017, 1033, 2041, 2049, 4095, 9001]
+
+
+def _bits(t):
+    return t.view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+
+
+def _want(x, bs, u=None):
+    return torch.from_numpy(oracle.fake_quantize(x.float().numpy(), bs, u)).to(x.dtype)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("cols", COLS)
+def test_fq_ragged_rows(cols, dt):
+    from axs.unified.hip_kernels import hip_fused_fake_quantize
+
+    g = torch.Generator().manual_seed(cols)
+    for rows, bs in ((1, 32), (3, 8), (37, 32), (50, 16)):
+        x = (torch.randn(rows, cols, generator=g) * torch.exp2(torch.randint(-8, 8, (rows, 1), generator=g))).to(dt)
+        x[0, : min(40, cols)] = 0.0
+        # one element into a buffer that ends with the tensor
+        buf = torch.empty(rows * cols + 1, dtype=dt, device=DEV)
+        xd = buf[1:].view(rows, cols).copy_(x)
+        for v in (x.to(DEV), xd):
+            got = hip_fused_fake_quantize(v, bs).cpu()
+            assert torch.equal(_bits(got), _bits(_want(x, bs))), (rows, bs)
+        u = oracle.uniform(SEED, 0, x.numel())
+        got = hip_fused_fake_quantize(xd, bs, "stochastic", seed=SEED).cpu()
+        assert torch.equal(_bits(got), _bits(_want(x, bs, u))), (rows, bs)
