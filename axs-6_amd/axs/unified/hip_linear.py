@@ -118,17 +118,13 @@ def _bias_vector(bias, N: int, fn: str):
     return bias.reshape(N).to(torch.float32).contiguous()
 
 
-def _as_input_dtype(out: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """Y in the input's floating dtype (float64 is computed in float32 and
-    returned as float64, as the reference's F.linear on its FQ values)."""
-    return out.to(dtype) if out.dtype != dtype and dtype.is_floating_point else out
-
-
 def fused_forward(input, weight, bias=None, quantize_input=True):
     """``FQ(input) FQ(weight)^T + bias`` with block size 32 in one launch of
     the fused kernel (FQ in the tile loads, fp32 contraction): the
     reference's ``triton_fused_linear`` (``triton_kernels.py:385-482``).
-    Returns the input's dtype (other floating dtypes are computed in float32)."""
+    Returns the input's dtype (other floating dtypes are computed in float32).
+    The host side is the extension's (axs._C.fused_linear): from Python the call
+    cost 13-22 us of host time, as much as most of its launches run."""
     fn = "axs_fused_linear"
     _require_device(input, fn)
     _require_device(weight, fn)
@@ -137,32 +133,7 @@ def fused_forward(input, weight, bias=None, quantize_input=True):
     N, Kw = weight.shape
     if Kw != K:
         raise RuntimeError(f"{fn}: input has {K} features but weight expects {Kw}")
-    b = _bias_vector(bias, N, fn)
-    dtype = input.dtype if input.dtype in _SUPPORTED else torch.float32
-    x2 = _dense(_pad_last(_rows(input, K).to(dtype), 32))
-    w2 = _dense(_pad_last(weight.to(dtype), 32))
-    M, Kb = x2.shape
-    dev = x2.device
-    y = torch.empty((M, N), dtype=dtype, device=dev)
-    if M and N and not Kb:
-        y.copy_(b.to(dtype).expand(M, N) if b is not None else torch.zeros((), dtype=dtype, device=dev).expand(M, N))
-    elif M and N:
-        code = _lib.DTYPE_CODE[dtype]
-        qx = bool(quantize_input)
-        with _on_device(x2):
-            st = _lib.stream_of(x2)
-            if _lib.lib().axs6_nf5_fused_linear_split_x(M, N, Kb, code):
-                # FQ(X) written once in the contraction's read order, then the
-                # contraction on it: the same values, where the single launch
-                # would read and quantize all of X in every workgroup
-                xa = torch.empty(_lib.lib().axs6_nf5_fused_linear_split_workspace(M, Kb) // 4,
-                                 dtype=torch.float32, device=dev)
-                _lib.call("axs6_nf5_fused_linear_split", x2.data_ptr(), w2.data_ptr(), _lib.ptr(b), y.data_ptr(),
-                          xa.data_ptr(), code, M, N, Kb, 32, int(qx), st)
-            else:
-                _lib.call("axs6_nf5_fused_linear", x2.data_ptr(), w2.data_ptr(), _lib.ptr(b), y.data_ptr(),
-                          code, M, N, Kb, 32, int(qx), st)
-    return _as_input_dtype(y.reshape(*input.shape[:-1], N), input.dtype)
+    return _lib.ext().fused_linear(input, weight, _bias_vector(bias, N, fn), bool(quantize_input))
 
 
 def linear_forward(input, weight, bias=None, block_size=32, quantize_input=True):

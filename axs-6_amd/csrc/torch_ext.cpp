@@ -423,6 +423,53 @@ at::Tensor linear(const at::Tensor& input, const at::Tensor& weight, const std::
                                  quantize_input, quantize_grad, has_bias, train);
 }
 
+// axs6_nf5_fused_linear (axs/unified/triton_kernels.py:385-482) for input (*, K)
+// and weight (N, K) of at most 128K outputs, block size 32: FQ values in
+// float32, one launch, or two where the library advises it.  K off the block is
+// zero-padded; the result has the input's dtype.  The caller has checked devices.
+at::Tensor fused_linear(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
+                        bool quantize_input) {
+    const char* fn = "axs_fused_linear";
+    require_device(input, fn);
+    require_device(weight, fn);
+    TORCH_CHECK(weight.device() == input.device() &&
+                    (!bias || !bias->defined() || bias->device() == input.device()),
+                fn, ": operands on different devices");
+    TORCH_CHECK(input.dim() >= 1 && weight.dim() == 2, fn, ": expected input (*, K) and weight (N, K)");
+    const int64_t K = input.size(-1), N = weight.size(0);
+    TORCH_CHECK(weight.size(1) == K, fn, ": input has ", K, " features but weight expects ", weight.size(1));
+    at::Tensor b;
+    if (bias && bias->defined()) b = bias_vector(*bias, N, fn).to(at::kFloat).contiguous();
+    const at::ScalarType dtype = compute_dtype(input.scalar_type());
+    const int code = dtype_code(dtype);
+    at::Tensor x2 = dense(pad_last(rows2d(input, K).to(dtype), 32));
+    at::Tensor w2 = dense(pad_last(weight.to(dtype), 32));
+    const int64_t M = x2.size(0), Kb = x2.size(1);
+    at::Tensor y = at::empty({M, N}, x2.options());
+    if (M && N && !Kb) {
+        if (b.defined()) y.copy_(b.to(dtype).expand({M, N}));
+        else y.zero_();
+    } else if (M && N) {
+        c10::DeviceGuard guard(x2.device());
+        const float* bp = b.defined() ? b.data_ptr<float>() : nullptr;
+        if (axs6_nf5_fused_linear_split_x(M, N, Kb, code)) {
+            // FQ(X) written once in the contraction's read order, then the
+            // contraction on it: the same values, where the single launch
+            // would read and quantize all of X in every workgroup
+            at::Tensor xa = at::empty({axs6_nf5_fused_linear_split_workspace(M, Kb) / 4},
+                                      x2.options().dtype(at::kFloat));
+            check_rc(axs6_nf5_fused_linear_split(x2.data_ptr(), w2.data_ptr(), bp, y.data_ptr(), xa.data_ptr<float>(),
+                                                 code, M, N, Kb, 32, quantize_input ? 1 : 0, stream_of(x2)),
+                     "axs6_nf5_fused_linear_split");
+        } else {
+            check_rc(axs6_nf5_fused_linear(x2.data_ptr(), w2.data_ptr(), bp, y.data_ptr(), code, M, N, Kb, 32,
+                                           quantize_input ? 1 : 0, stream_of(x2)),
+                     "axs6_nf5_fused_linear");
+        }
+    }
+    return to_input_dtype(y.reshape(lead_shape(input.sizes(), N)), input.scalar_type());
+}
+
 // The forward alone, no gradient recorded.
 at::Tensor linear_infer(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
                         int64_t bs, bool quantize_input) {
@@ -533,6 +580,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("linear", &linear, "FQ(input) FQ(weight)^T + bias with the quantized backward (autograd node)",
           py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("block_size"), py::arg("quantize_input"),
           py::arg("quantize_grad"));
+    m.def("fused_linear", &fused_linear, "the fused linear of small outputs (block size 32, no autograd)",
+          py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("quantize_input"));
     m.def("linear_infer", &linear_infer, "the forward alone: FQ(input) FQ(weight)^T + bias (no autograd)",
           py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("block_size"), py::arg("quantize_input"));
     m.def("linear_fwd", &linear_fwd,
