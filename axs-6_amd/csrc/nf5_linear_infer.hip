@@ -253,7 +253,6 @@ __device__ __forceinline__ f32x4m mfma_elem(u32x4 a, u32x4 b, f32x4m c) {
 }
 
 constexpr int kXSlabs = 3;
-constexpr int kWRing = 2;                // K steps of raw weight values in flight
 template <int DT, int BM> constexpr int infer_waves() { return BM >= 128 || (DT == AXS6_F32 && BM == 64) ? 2 : 4; }
 
 constexpr size_t infer_lds(int BM) {
@@ -379,7 +378,7 @@ __global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm
     constexpr int XINST = BM / 8;                    // 1 KiB DMA instructions per X slab
     constexpr int XI = XINST >= 8 ? XINST / 8 : 1;   // per (issuing) wave
     constexpr int WI = 2 * RV;
-    constexpr int D = kWRing;
+    constexpr int D = 2;                             // K steps of raw weight values in flight
     extern __shared__ __align__(16) char smem[];
     __shared__ InferTables tab;
     char* const xs = smem;
