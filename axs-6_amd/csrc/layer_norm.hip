@@ -65,11 +65,29 @@ __device__ __forceinline__ void load_vec(const void* p, int64_t i, float* f) {
     E::unpack(reinterpret_cast<const u32x4*>(p)[i], f);
 }
 
-template <int DT>
-__device__ __forceinline__ void store_vec(void* p, int64_t i, const float* f) {
-    using E = Elem<DT>;
-    reinterpret_cast<u32x4*>(p)[i] = E::pack(f);
+// One vector's raw words, and a store, with the nontemporal hint when NT.
+template <int DT, bool NT>
+__device__ __forceinline__ u32x4 load_raw(const void* p, int64_t i) {
+    if constexpr (NT) return ld_stream(reinterpret_cast<const u32x4*>(p) + i);
+    else return reinterpret_cast<const u32x4*>(p)[i];
 }
+template <int DT, bool NT>
+__device__ __forceinline__ void store_vec_hint(void* p, int64_t i, const float* f) {
+    if constexpr (NT) st_stream(Elem<DT>::pack(f), reinterpret_cast<u32x4*>(p) + i);
+    else reinterpret_cast<u32x4*>(p)[i] = Elem<DT>::pack(f);
+}
+
+// Tensors of this many bytes and more stream: y and dx by nontemporal stores,
+// and the backward's x and dy, read for the last time, by nontemporal loads
+// (the forward's x by plain ones: a backward reads it again).  Plain stores
+// leave the 256 MiB last-level cache dirty lines whose write-back the next
+// kernels pay.  us, forward and forward + backward, three tensors in turn,
+// plain -> streaming: 8192 x 4096 f32 53.5, 143.0 -> 50.3, 118.7; 16384 x 2048
+// f32 49.2, 137.8 -> 48.3, 117.7; 8192 x 4096 bf16 32.2, 95.5 -> 22.5, 85.8;
+// 8192 x 1024 f32 12.5, 39.2 -> 12.1, 33.4.  Below, a tensor stays in the cache
+// for what reads it next, and streaming loads lose (8192 x 1024 bf16, 16 MiB:
+// 27.9 -> 29.9).
+constexpr int64_t kLnStreamBytes = (int64_t)32 << 20;
 
 struct LnArgs {
     const void* x; const void* dy; const void* gamma; const void* beta;
@@ -84,7 +102,7 @@ struct LnArgs {
 // NT threads per row, NV 16-byte vectors each; RPW rows per workgroup
 // (RPW > 1 only with NT == 64).  Thread t of a row group holds vectors
 // t, t + NT, ..., t + (NV - 1) * NT of the row.
-template <int DT, int NT, int NV>
+template <int DT, int NT, int NV, bool STREAM>
 __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
     using E = Elem<DT>;
     constexpr int V = E::V, RPW = kLnThreads / NT;
@@ -159,7 +177,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
                 }
 #pragma unroll
                 for (int e = 0; e < V; ++e) o[e] = (v[j][e] - mean) * rstd * gw[e] + bw[e];
-                store_vec<DT>(yr, vi, o);
+                store_vec_hint<DT, STREAM>(yr, vi, o);
             }
         }
         if (t == 0) {
@@ -169,7 +187,11 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
     }
 }
 
-template <int DT, int NT, int NV>
+// PF: the next row's x and dy are loaded while a row is reduced (two barriers)
+// and written.  Forward + backward, us, without -> with: 8192 x 4096 bf16 86.3
+// -> 76.3, 4096 x 8192 bf16 93.0 -> 82.2, 4096 x 8192 f32 128.7 -> 123.1; shorter
+// f32 rows have enough workgroups in flight and lose (8192 x 4096 119.8 -> 123).
+template <int DT, int NT, int NV, bool STREAM>
 __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     using E = Elem<DT>;
     constexpr int V = E::V, RPW = kLnThreads / NT;
@@ -187,24 +209,44 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     }
     const float inv_n = 1.0f / (float)a.cols;
     const size_t es = sizeof(typename E::S);
-    for (int64_t r0 = (int64_t)blockIdx.x * RPW; r0 < a.rows; r0 += (int64_t)gridDim.x * RPW) {
+    constexpr bool PF = DT != AXS6_F32 || NV >= 6;
+    u32x4 nx[NV], nd[NV];
+    float nmean = 0.0f, nrstd = 0.0f;
+    // a row past the last reads the last; columns past the row read its last vector
+    auto fetch = [&](int64_t row) {
+        const int64_t r = row < a.rows ? row : a.rows - 1;
+        const char* xr = reinterpret_cast<const char*>(a.x) + r * a.cols * (int64_t)es;
+        const char* dyr = reinterpret_cast<const char*>(a.dy) + r * a.cols * (int64_t)es;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int64_t vi = t + (int64_t)j * NT, vc = vi < nvec ? vi : nvec - 1;
+            nx[j] = load_raw<DT, STREAM>(xr, vc);
+            nd[j] = load_raw<DT, STREAM>(dyr, vc);
+        }
+        nmean = a.mean[r];
+        nrstd = a.rstd[r];
+    };
+    const int64_t rstep = (int64_t)gridDim.x * RPW;
+    if constexpr (PF) fetch((int64_t)blockIdx.x * RPW + g);
+    for (int64_t r0 = (int64_t)blockIdx.x * RPW; r0 < a.rows; r0 += rstep) {
         const int64_t r = r0 + g;
         if (NT == 64 && r >= a.rows) break;
-        const void* xr = reinterpret_cast<const char*>(a.x) + r * a.cols * (int64_t)es;
-        const void* dyr = reinterpret_cast<const char*>(a.dy) + r * a.cols * (int64_t)es;
-        const float mean = a.mean[r], rstd = a.rstd[r];
+        if constexpr (!PF) fetch(r);
+        const float mean = nmean, rstd = nrstd;
+        u32x4 cx[NV], cd[NV];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) { cx[j] = nx[j]; cd[j] = nd[j]; }
+        if constexpr (PF) fetch(r + rstep);
         float xh[NV][V], gg[NV][V];
         float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int64_t vi = t + (int64_t)j * NT;
             float xv[V], dv[V];
+            E::unpack(cx[j], xv);
+            E::unpack(cd[j], dv);
 #pragma unroll
-            for (int e = 0; e < V; ++e) { xv[e] = 0.0f; dv[e] = 0.0f; }
-            if (vi < nvec) {
-                load_vec<DT>(xr, vi, xv);
-                load_vec<DT>(dyr, vi, dv);
-            }
+            for (int e = 0; e < V; ++e) dv[e] = vi < nvec ? dv[e] : 0.0f;
             const bool in = vi < nvec;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
@@ -225,7 +267,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
                 float o[V];
 #pragma unroll
                 for (int e = 0; e < V; ++e) o[e] = rstd * (gg[j][e] - (s.x + xh[j][e] * s.y) * inv_n);
-                store_vec<DT>(dxr, vi, o);
+                store_vec_hint<DT, STREAM>(dxr, vi, o);
             }
         }
     }
@@ -393,17 +435,24 @@ LnShape ln_shape(int dtype, int64_t cols, const void* const* ptrs, int nptr, boo
     return s;
 }
 
+template <int DT>
+bool ln_streams(const LnArgs& a) {
+    return a.rows * a.cols * (int64_t)sizeof(typename Elem<DT>::S) >= kLnStreamBytes;
+}
+
 template <int DT, int NT, int NV>
 void launch_fwd_vec(const LnArgs& a, hipStream_t st) {
     constexpr int RPW = kLnThreads / NT;
     const int64_t groups = (a.rows + RPW - 1) / RPW;
     const unsigned grid = (unsigned)(groups < 65536 ? groups : 65536);
-    ln_fwd_vec_kernel<DT, NT, NV><<<grid, kLnThreads, 0, st>>>(a);
+    if (ln_streams<DT>(a)) ln_fwd_vec_kernel<DT, NT, NV, true><<<grid, kLnThreads, 0, st>>>(a);
+    else ln_fwd_vec_kernel<DT, NT, NV, false><<<grid, kLnThreads, 0, st>>>(a);
 }
 
 template <int DT, int NT, int NV>
 void launch_bwd_vec(const LnArgs& a, int64_t chunks, hipStream_t st) {
-    ln_bwd_vec_kernel<DT, NT, NV><<<(unsigned)chunks, kLnThreads, 0, st>>>(a);
+    if (ln_streams<DT>(a)) ln_bwd_vec_kernel<DT, NT, NV, true><<<(unsigned)chunks, kLnThreads, 0, st>>>(a);
+    else ln_bwd_vec_kernel<DT, NT, NV, false><<<(unsigned)chunks, kLnThreads, 0, st>>>(a);
 }
 
 template <int DT>
