@@ -10,22 +10,29 @@
 //   backward (g = dy * gamma):  dx = rstd_r * (g - (sum_c g + xhat * sum_c g*xhat) / cols),
 //   dgamma[c] = sum_r dy * xhat,  dbeta[c] = sum_r dy
 //
-// Vector form (rows of whole 16-byte vectors, 16-byte aligned, at most
-// 8192 f32 / 16384 16-bit values): a row is held in registers -- one wave per
-// row up to 1024 f32 / 2048 16-bit values (four rows per workgroup), else
-// one 256-thread workgroup per row -- so the statistics take one HBM read.
+// Vector form (rows of one 16-byte vector to 8192 values): a row is held in
+// registers -- one wave per row up to 1024 f32 / 2048 16-bit values (1024 in
+// the backward; four rows per workgroup), else one 256-thread workgroup per
+// row -- so the statistics take one HBM read.  Rows that are not whole vectors,
+// and unaligned tensors, take the same form with unaligned 16-byte accesses
+// (RAG); a ragged row's last vector overlaps the one before.  Against the
+// generic form, which reads a value per lane and each row two or three times,
+// forward + backward, us: 8192 x 1001 bf16 64 -> 33, 8192 x 999 f32 60 -> 38,
+// 2048 x 4095 f32 64 -> 48 (whole vectors: 8192 x 1000 bf16 30).
 // The backward reads x and dy once per row: each thread keeps its columns'
 // dgamma/dbeta sums over the rows of its workgroup, the workgroup writes them
 // as one partial row (dgamma rows, then dbeta rows, one per workgroup), and a
 // second launch sums the partial rows in a fixed order (deterministic for a
 // given shape).
 //
-// Generic form (any length, alignment or size): one 256-thread workgroup per
-// row streams it (three passes forward, two backward; the passes after the
-// first read the row back from cache); the parameter sums run as a column
-// pass over row ranges (one partial row per range) before the same fixed-order
-// reduction.
+// Generic form (rows longer than that or shorter than a vector): one
+// 256-thread workgroup per row streams it (three passes forward, two backward;
+// the passes after the first read the row back from cache); the parameter sums
+// run as a column pass over row ranges (one partial row per range) before the
+// same fixed-order reduction.
 #include <math.h>
+
+#include <type_traits>
 
 #include "axs6_internal.h"
 #include "nf5_device.h"
@@ -59,22 +66,43 @@ __device__ __forceinline__ float2 group_sum2(float a, float b, float* red) {
     }
 }
 
-template <int DT>
+// A 16-byte vector at element i of p: aligned, or (RAG) at any element's
+// address, still one load or store; with the nontemporal hint when NT.
+typedef u32x4 u32x4_el2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_el4 __attribute__((aligned(4)));
+template <int DT, bool RAG>
+using VecAt = std::conditional_t<!RAG, u32x4, std::conditional_t<DT == AXS6_F32, u32x4_el4, u32x4_el2>>;
+
+template <int DT, bool NT, bool RAG>
+__device__ __forceinline__ u32x4 load_raw(const void* p, int64_t i) {
+    const auto* q = reinterpret_cast<const VecAt<DT, RAG>*>(reinterpret_cast<const typename Elem<DT>::S*>(p) + i);
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
+}
+template <int DT, bool RAG>
 __device__ __forceinline__ void load_vec(const void* p, int64_t i, float* f) {
-    using E = Elem<DT>;
-    E::unpack(reinterpret_cast<const u32x4*>(p)[i], f);
+    Elem<DT>::unpack(load_raw<DT, false, RAG>(p, i), f);
+}
+template <int DT, bool NT, bool RAG>
+__device__ __forceinline__ void store_vec(void* p, int64_t i, const float* f) {
+    auto* q = reinterpret_cast<VecAt<DT, RAG>*>(reinterpret_cast<typename Elem<DT>::S*>(p) + i);
+    if constexpr (NT) __builtin_nontemporal_store(Elem<DT>::pack(f), q);
+    else *q = Elem<DT>::pack(f);
 }
 
-// One vector's raw words, and a store, with the nontemporal hint when NT.
-template <int DT, bool NT>
-__device__ __forceinline__ u32x4 load_raw(const void* p, int64_t i) {
-    if constexpr (NT) return ld_stream(reinterpret_cast<const u32x4*>(p) + i);
-    else return reinterpret_cast<const u32x4*>(p)[i];
+// First element of a row's vector vi (vi < nvec).  A ragged row's last vector
+// starts before its place so that it ends with the row: the elements it shares
+// with the one before are left out of the sums (vec_own) and written by both
+// lanes with the same bits.
+template <int V, bool RAG>
+__device__ __forceinline__ int64_t vec_at(int64_t vi, int64_t cols) {
+    const int64_t o = vi * V;
+    if constexpr (RAG) return o < cols - V ? o : cols - V;
+    else return o;
 }
-template <int DT, bool NT>
-__device__ __forceinline__ void store_vec_hint(void* p, int64_t i, const float* f) {
-    if constexpr (NT) st_stream(Elem<DT>::pack(f), reinterpret_cast<u32x4*>(p) + i);
-    else reinterpret_cast<u32x4*>(p)[i] = Elem<DT>::pack(f);
+template <int V, bool RAG>
+__device__ __forceinline__ bool vec_own(int64_t vi, int64_t at, int e) {
+    return !RAG || at + e >= vi * V;
 }
 
 // Tensors of this many bytes and more stream: y and dx by nontemporal stores,
@@ -102,13 +130,13 @@ struct LnArgs {
 // NT threads per row, NV 16-byte vectors each; RPW rows per workgroup
 // (RPW > 1 only with NT == 64).  Thread t of a row group holds vectors
 // t, t + NT, ..., t + (NV - 1) * NT of the row.
-template <int DT, int NT, int NV, bool STREAM>
+template <int DT, int NT, int NV, bool STREAM, bool RAG>
 __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
     using E = Elem<DT>;
     constexpr int V = E::V, RPW = kLnThreads / NT;
     __shared__ float red[8];
     const int t = threadIdx.x % NT, g = threadIdx.x / NT;
-    const int64_t nvec = a.cols / V;
+    const int64_t nvec = (a.cols + V - 1) / V;
     // a wave's row group keeps its columns' gamma and beta in registers across
     // rows; a workgroup row reads them at the store (cache hits), which leaves
     // registers for more rows in flight
@@ -122,8 +150,9 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
 #pragma unroll
             for (int e = 0; e < V; ++e) { gm[j][e] = 1.0f; bt[j][e] = 0.0f; }
             if (vi < nvec) {
-                if (a.gamma) load_vec<DT>(a.gamma, vi, gm[j]);
-                if (a.beta) load_vec<DT>(a.beta, vi, bt[j]);
+                const int64_t at = vec_at<V, RAG>(vi, a.cols);
+                if (a.gamma) load_vec<DT, RAG>(a.gamma, at, gm[j]);
+                if (a.beta) load_vec<DT, RAG>(a.beta, at, bt[j]);
             }
         }
     }
@@ -142,20 +171,22 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
 #pragma unroll
             for (int e = 0; e < V; ++e) v[j][e] = 0.0f;
             if (vi < nvec) {
-                load_vec<DT>(xr, vi, v[j]);
+                const int64_t at = vec_at<V, RAG>(vi, a.cols);
+                load_vec<DT, RAG>(xr, at, v[j]);
 #pragma unroll
-                for (int e = 0; e < V; ++e) s += v[j][e] - piv;
+                for (int e = 0; e < V; ++e) s += vec_own<V, RAG>(vi, at, e) ? v[j][e] - piv : 0.0f;
             }
         }
         const float mean = piv + group_sum2<NT>(s, 0.0f, red).x / (float)a.cols;
         float q = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            const bool in = t + (int64_t)j * NT < nvec;
+            const int64_t vi = t + (int64_t)j * NT, at = vec_at<V, RAG>(vi, a.cols);
+            const bool in = vi < nvec;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 const float d = v[j][e] - mean;
-                q += in ? d * d : 0.0f;
+                q += in && vec_own<V, RAG>(vi, at, e) ? d * d : 0.0f;
             }
         }
         const float var = group_sum2<NT>(q, 0.0f, red).x / (float)a.cols;
@@ -165,6 +196,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
         for (int j = 0; j < NV; ++j) {
             const int64_t vi = t + (int64_t)j * NT;
             if (vi < nvec) {
+                const int64_t at = vec_at<V, RAG>(vi, a.cols);
                 float o[V], gw[V], bw[V];
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
@@ -172,12 +204,12 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
                     bw[e] = KEEP ? bt[KEEP ? j : 0][e] : 0.0f;
                 }
                 if constexpr (!KEEP) {
-                    if (a.gamma) load_vec<DT>(a.gamma, vi, gw);
-                    if (a.beta) load_vec<DT>(a.beta, vi, bw);
+                    if (a.gamma) load_vec<DT, RAG>(a.gamma, at, gw);
+                    if (a.beta) load_vec<DT, RAG>(a.beta, at, bw);
                 }
 #pragma unroll
                 for (int e = 0; e < V; ++e) o[e] = (v[j][e] - mean) * rstd * gw[e] + bw[e];
-                store_vec_hint<DT, STREAM>(yr, vi, o);
+                store_vec<DT, STREAM, RAG>(yr, at, o);
             }
         }
         if (t == 0) {
@@ -191,21 +223,21 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
 // and written.  Forward + backward, us, without -> with: 8192 x 4096 bf16 86.3
 // -> 76.3, 4096 x 8192 bf16 93.0 -> 82.2, 4096 x 8192 f32 128.7 -> 123.1; shorter
 // f32 rows have enough workgroups in flight and lose (8192 x 4096 119.8 -> 123).
-template <int DT, int NT, int NV, bool STREAM>
+template <int DT, int NT, int NV, bool STREAM, bool RAG>
 __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     using E = Elem<DT>;
     constexpr int V = E::V, RPW = kLnThreads / NT;
     __shared__ float red[8];
     __shared__ float cs[RPW > 1 ? RPW : 1][2][64 * V + 1];   // per-wave column sums (NT == 64)
     const int t = threadIdx.x % NT, g = threadIdx.x / NT;
-    const int64_t nvec = a.cols / V;
+    const int64_t nvec = (a.cols + V - 1) / V;
     float gm[NV][V], pg[NV][V], pb[NV][V];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int64_t vi = t + (int64_t)j * NT;
 #pragma unroll
         for (int e = 0; e < V; ++e) { gm[j][e] = 1.0f; pg[j][e] = 0.0f; pb[j][e] = 0.0f; }
-        if (a.gamma && vi < nvec) load_vec<DT>(a.gamma, vi, gm[j]);
+        if (a.gamma && vi < nvec) load_vec<DT, RAG>(a.gamma, vec_at<V, RAG>(vi, a.cols), gm[j]);
     }
     const float inv_n = 1.0f / (float)a.cols;
     const size_t es = sizeof(typename E::S);
@@ -219,9 +251,9 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
         const char* dyr = reinterpret_cast<const char*>(a.dy) + r * a.cols * (int64_t)es;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            const int64_t vi = t + (int64_t)j * NT, vc = vi < nvec ? vi : nvec - 1;
-            nx[j] = load_raw<DT, STREAM>(xr, vc);
-            nd[j] = load_raw<DT, STREAM>(dyr, vc);
+            const int64_t vi = t + (int64_t)j * NT, at = vec_at<V, RAG>(vi < nvec ? vi : nvec - 1, a.cols);
+            nx[j] = load_raw<DT, STREAM, RAG>(xr, at);
+            nd[j] = load_raw<DT, STREAM, RAG>(dyr, at);
         }
         nmean = a.mean[r];
         nrstd = a.rstd[r];
@@ -241,7 +273,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
         float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            const int64_t vi = t + (int64_t)j * NT;
+            const int64_t vi = t + (int64_t)j * NT, at = vec_at<V, RAG>(vi, a.cols);
             float xv[V], dv[V];
             E::unpack(cx[j], xv);
             E::unpack(cd[j], dv);
@@ -252,8 +284,9 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
             for (int e = 0; e < V; ++e) {
                 xh[j][e] = in ? (xv[e] - mean) * rstd : 0.0f;   // dy is 0 past the row too
                 gg[j][e] = dv[e] * gm[j][e];
-                s1 += gg[j][e];
-                s2 += gg[j][e] * xh[j][e];
+                const float go = vec_own<V, RAG>(vi, at, e) ? gg[j][e] : 0.0f;
+                s1 += go;
+                s2 += vec_own<V, RAG>(vi, at, e) ? gg[j][e] * xh[j][e] : 0.0f;
                 pg[j][e] += dv[e] * xh[j][e];
                 pb[j][e] += dv[e];
             }
@@ -267,7 +300,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
                 float o[V];
 #pragma unroll
                 for (int e = 0; e < V; ++e) o[e] = rstd * (gg[j][e] - (s.x + xh[j][e] * s.y) * inv_n);
-                store_vec_hint<DT, STREAM>(dxr, vi, o);
+                store_vec<DT, STREAM, RAG>(dxr, vec_at<V, RAG>(vi, a.cols), o);
             }
         }
     }
@@ -277,23 +310,27 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     if constexpr (RPW == 1) {
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            const int64_t vi = t + (int64_t)j * NT;
+            const int64_t vi = t + (int64_t)j * NT, at = vec_at<V, RAG>(vi, a.cols);
             if (vi < nvec) {
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
-                    prow[0][vi * V + e] = pg[j][e];
-                    prow[1][vi * V + e] = pb[j][e];
+                    if (!vec_own<V, RAG>(vi, at, e)) continue;
+                    prow[0][at + e] = pg[j][e];
+                    prow[1][at + e] = pb[j][e];
                 }
             }
         }
     } else {
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
+            const int64_t vi = t + (int64_t)j * NT, at = vec_at<V, RAG>(vi, a.cols);
+            const int c0 = RAG ? (int)(at - (int64_t)j * 64 * V) : t * V;
             __syncthreads();
 #pragma unroll
             for (int e = 0; e < V; ++e) {
-                cs[g][0][t * V + e] = pg[j][e];
-                cs[g][1][t * V + e] = pb[j][e];
+                if (RAG && !(vi < nvec && vec_own<V, RAG>(vi, at, e))) continue;
+                cs[g][0][c0 + e] = pg[j][e];
+                cs[g][1][c0 + e] = pb[j][e];
             }
             __syncthreads();
             // thread k of the workgroup adds column k % (64 V) of the staged
@@ -406,22 +443,22 @@ __global__ __launch_bounds__(kLnThreads) void ln_reduce_kernel(const float* part
 
 // ---- launch shapes ---------------------------------------------------------------
 
-struct LnShape { int nt; int nv; bool vec; };
+struct LnShape { int nt; int nv; bool vec; bool ragged; };
 
 // Row groups of 64 threads (one wave per row) while a row has at most
 // 64 * cap64 vectors, else 256 threads with at most cap256 vectors each;
-// longer, ragged or unaligned rows take the generic form.  The caps keep the
+// longer rows and rows shorter than a vector take the generic form.  The caps keep the
 // row in registers without spills (the backward holds five values per
 // element, 16-bit rows twice as many elements per vector).
 LnShape ln_shape(int dtype, int64_t cols, const void* const* ptrs, int nptr, bool bwd) {
     const int V = dtype == AXS6_F32 ? 4 : 8;
     const int cap64 = (bwd && V == 8) ? 2 : 4;
     const int cap256 = (V == 8) ? 4 : 8;
-    LnShape s{0, 0, false};
-    if (cols <= 0 || cols % V != 0) return s;
+    LnShape s{0, 0, false, cols % V != 0};
+    if (cols < V) return s;
     for (int i = 0; i < nptr; ++i)
-        if (ptrs[i] && (uintptr_t)ptrs[i] % 16 != 0) return s;
-    const int64_t nvec = cols / V;
+        if (ptrs[i] && (uintptr_t)ptrs[i] % 16 != 0) s.ragged = true;
+    const int64_t nvec = (cols + V - 1) / V;
     if (nvec <= 64 * cap64) {
         s.nt = 64;
         s.nv = (int)((nvec + 63) / 64);
@@ -441,18 +478,31 @@ bool ln_streams(const LnArgs& a) {
 }
 
 template <int DT, int NT, int NV>
-void launch_fwd_vec(const LnArgs& a, hipStream_t st) {
+void launch_fwd_vec(const LnArgs& a, const LnShape& s, hipStream_t st) {
     constexpr int RPW = kLnThreads / NT;
     const int64_t groups = (a.rows + RPW - 1) / RPW;
     const unsigned grid = (unsigned)(groups < 65536 ? groups : 65536);
-    if (ln_streams<DT>(a)) ln_fwd_vec_kernel<DT, NT, NV, true><<<grid, kLnThreads, 0, st>>>(a);
-    else ln_fwd_vec_kernel<DT, NT, NV, false><<<grid, kLnThreads, 0, st>>>(a);
+    const bool nt = ln_streams<DT>(a);
+    if (s.ragged) {
+        if (nt) ln_fwd_vec_kernel<DT, NT, NV, true, true><<<grid, kLnThreads, 0, st>>>(a);
+        else ln_fwd_vec_kernel<DT, NT, NV, false, true><<<grid, kLnThreads, 0, st>>>(a);
+    } else {
+        if (nt) ln_fwd_vec_kernel<DT, NT, NV, true, false><<<grid, kLnThreads, 0, st>>>(a);
+        else ln_fwd_vec_kernel<DT, NT, NV, false, false><<<grid, kLnThreads, 0, st>>>(a);
+    }
 }
 
 template <int DT, int NT, int NV>
-void launch_bwd_vec(const LnArgs& a, int64_t chunks, hipStream_t st) {
-    if (ln_streams<DT>(a)) ln_bwd_vec_kernel<DT, NT, NV, true><<<(unsigned)chunks, kLnThreads, 0, st>>>(a);
-    else ln_bwd_vec_kernel<DT, NT, NV, false><<<(unsigned)chunks, kLnThreads, 0, st>>>(a);
+void launch_bwd_vec(const LnArgs& a, const LnShape& s, int64_t chunks, hipStream_t st) {
+    const bool nt = ln_streams<DT>(a);
+    const unsigned grid = (unsigned)chunks;
+    if (s.ragged) {
+        if (nt) ln_bwd_vec_kernel<DT, NT, NV, true, true><<<grid, kLnThreads, 0, st>>>(a);
+        else ln_bwd_vec_kernel<DT, NT, NV, false, true><<<grid, kLnThreads, 0, st>>>(a);
+    } else {
+        if (nt) ln_bwd_vec_kernel<DT, NT, NV, true, false><<<grid, kLnThreads, 0, st>>>(a);
+        else ln_bwd_vec_kernel<DT, NT, NV, false, false><<<grid, kLnThreads, 0, st>>>(a);
+    }
 }
 
 template <int DT>
@@ -464,24 +514,24 @@ int fwd_dispatch(const LnArgs& a, const LnShape& s, hipStream_t st) {
     }
     if (s.nt == 64) {
         switch (s.nv) {
-            case 1: launch_fwd_vec<DT, 64, 1>(a, st); break;
-            case 2: launch_fwd_vec<DT, 64, 2>(a, st); break;
-            case 3: launch_fwd_vec<DT, 64, 3>(a, st); break;
-            default: launch_fwd_vec<DT, 64, 4>(a, st); break;
+            case 1: launch_fwd_vec<DT, 64, 1>(a, s, st); break;
+            case 2: launch_fwd_vec<DT, 64, 2>(a, s, st); break;
+            case 3: launch_fwd_vec<DT, 64, 3>(a, s, st); break;
+            default: launch_fwd_vec<DT, 64, 4>(a, s, st); break;
         }
     } else if constexpr (DT == AXS6_F32) {
         switch (s.nv) {
-            case 1: case 2: launch_fwd_vec<DT, 256, 2>(a, st); break;
-            case 3: launch_fwd_vec<DT, 256, 3>(a, st); break;
-            case 4: launch_fwd_vec<DT, 256, 4>(a, st); break;
-            case 5: case 6: launch_fwd_vec<DT, 256, 6>(a, st); break;
-            default: launch_fwd_vec<DT, 256, 8>(a, st); break;
+            case 1: case 2: launch_fwd_vec<DT, 256, 2>(a, s, st); break;
+            case 3: launch_fwd_vec<DT, 256, 3>(a, s, st); break;
+            case 4: launch_fwd_vec<DT, 256, 4>(a, s, st); break;
+            case 5: case 6: launch_fwd_vec<DT, 256, 6>(a, s, st); break;
+            default: launch_fwd_vec<DT, 256, 8>(a, s, st); break;
         }
     } else {
         switch (s.nv) {
-            case 1: case 2: launch_fwd_vec<DT, 256, 2>(a, st); break;
-            case 3: launch_fwd_vec<DT, 256, 3>(a, st); break;
-            default: launch_fwd_vec<DT, 256, 4>(a, st); break;
+            case 1: case 2: launch_fwd_vec<DT, 256, 2>(a, s, st); break;
+            case 3: launch_fwd_vec<DT, 256, 3>(a, s, st); break;
+            default: launch_fwd_vec<DT, 256, 4>(a, s, st); break;
         }
     }
     return AXS6_OK;
@@ -499,30 +549,30 @@ int bwd_dispatch(const LnArgs& a, const LnShape& s, int64_t chunks, hipStream_t 
     if constexpr (DT == AXS6_F32) {
         if (s.nt == 64) {
             switch (s.nv) {
-                case 1: launch_bwd_vec<DT, 64, 1>(a, chunks, st); break;
-                case 2: launch_bwd_vec<DT, 64, 2>(a, chunks, st); break;
-                case 3: launch_bwd_vec<DT, 64, 3>(a, chunks, st); break;
-                default: launch_bwd_vec<DT, 64, 4>(a, chunks, st); break;
+                case 1: launch_bwd_vec<DT, 64, 1>(a, s, chunks, st); break;
+                case 2: launch_bwd_vec<DT, 64, 2>(a, s, chunks, st); break;
+                case 3: launch_bwd_vec<DT, 64, 3>(a, s, chunks, st); break;
+                default: launch_bwd_vec<DT, 64, 4>(a, s, chunks, st); break;
             }
         } else {
             switch (s.nv) {
-                case 1: case 2: launch_bwd_vec<DT, 256, 2>(a, chunks, st); break;
-                case 3: launch_bwd_vec<DT, 256, 3>(a, chunks, st); break;
-                case 4: launch_bwd_vec<DT, 256, 4>(a, chunks, st); break;
-                case 5: case 6: launch_bwd_vec<DT, 256, 6>(a, chunks, st); break;
-                default: launch_bwd_vec<DT, 256, 8>(a, chunks, st); break;
+                case 1: case 2: launch_bwd_vec<DT, 256, 2>(a, s, chunks, st); break;
+                case 3: launch_bwd_vec<DT, 256, 3>(a, s, chunks, st); break;
+                case 4: launch_bwd_vec<DT, 256, 4>(a, s, chunks, st); break;
+                case 5: case 6: launch_bwd_vec<DT, 256, 6>(a, s, chunks, st); break;
+                default: launch_bwd_vec<DT, 256, 8>(a, s, chunks, st); break;
             }
         }
     } else {
         if (s.nt == 64) {
-            if (s.nv == 1) launch_bwd_vec<DT, 64, 1>(a, chunks, st);
-            else launch_bwd_vec<DT, 64, 2>(a, chunks, st);
+            if (s.nv == 1) launch_bwd_vec<DT, 64, 1>(a, s, chunks, st);
+            else launch_bwd_vec<DT, 64, 2>(a, s, chunks, st);
         } else {
             switch (s.nv) {
-                case 1: launch_bwd_vec<DT, 256, 1>(a, chunks, st); break;
-                case 2: launch_bwd_vec<DT, 256, 2>(a, chunks, st); break;
-                case 3: launch_bwd_vec<DT, 256, 3>(a, chunks, st); break;
-                default: launch_bwd_vec<DT, 256, 4>(a, chunks, st); break;
+                case 1: launch_bwd_vec<DT, 256, 1>(a, s, chunks, st); break;
+                case 2: launch_bwd_vec<DT, 256, 2>(a, s, chunks, st); break;
+                case 3: launch_bwd_vec<DT, 256, 3>(a, s, chunks, st); break;
+                default: launch_bwd_vec<DT, 256, 4>(a, s, chunks, st); break;
             }
         }
     }

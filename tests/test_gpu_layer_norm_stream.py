@@ -2,7 +2,7 @@
 more: nontemporal stores and last-use loads) and the backward's next-row
 prefetch, at the edges: just below and at 32 MiB, row counts that leave a
 partial chunk or fewer rows than workgroups, and rows whose last vector group
-is partial.  Against float64 F.layer_norm; the bars are those of the kernels'
+is partial; and the ragged instances (rows of no whole number of vectors).  Against float64 F.layer_norm; the bars are those of the kernels'
 other test (f32: rounding of sums of up to 16K terms; 16-bit: one rounding of
 the result)."""
 from __future__ import annotations
@@ -31,6 +31,17 @@ CASES = [
     (1, 2056, torch.bfloat16),       # prefetch past the only row
     (17, 8192, torch.float32),
     (5, 520, torch.float16),
+    # ragged rows: unaligned vectors, the last one overlapping its neighbour
+    (300, 5, torch.float32),         # two vectors sharing three values
+    (300, 9, torch.bfloat16),
+    (301, 15, torch.float16),        # sharing one value
+    (70, 257, torch.float32),
+    (33, 1027, torch.float32),       # a workgroup per row
+    (9, 8191, torch.float32),        # the longest ragged vector row
+    (31, 2047, torch.float16),
+    (9, 8191, torch.bfloat16),
+    (4100, 4097, torch.bfloat16),    # streamed
+    (16400, 515, torch.float32),     # streamed, a wave per row
 ]
 
 
