@@ -397,14 +397,27 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitReduceK k) {
 // fixed ~7 us per 256x256 f32 tile and CU, all of a short-K GEMM's runtime
 // when 32 CUs carry it; 128x128 tiles spread it over 4x the CUs, two
 // workgroups sharing a CU.
+// Over 512 tiles of 128x128, two per CU, begins their second round, and one
+// round of 256x256 tiles on part of the CUs is the faster: packed operands to
+// f32, us, 128x128 -> 256x256 (M x K x N): 3584 x 4096 x 4096 123-144 -> 101,
+// 2560 x 4096 x 4096 98 -> 82, 2176 x 4096 x 4096 (144 tiles) 96-104 -> 86-90,
+// 3072 x 11008 x 4096 267 -> 221, 2305 x 1024 x 4093 69 -> 41, 20000 x 256 x 450
+// 50 -> 26, 3584 x 512 x 4096 26 -> 24, 3072 x 128 x 4096 14.2 -> 13.8; at 512
+// (2048 x 4096 x 4096) the smaller tiles take 64 against 78.  A 16-bit output of
+// a short contraction stays with them: its no-gradient linear, 3000 x 512 x
+// 3000 bf16 30.4 against 31.3, 4096 x 768 x 3072 39.1 against 39.9, 2048 x 1024 x
+// 4800 41.9 against 42.0 (2304 x 2048 x 4096 73.7 against 69.2).
 enum GemmCfg { kCfgBig = 0, kCfgSmall = 1, kCfgNarrow = 2 };
+constexpr int64_t kBigShortK = 1024;
 constexpr int kNarrowDeepSteps = 32;   // 64-deep K-steps per workgroup from which narrow runs three slabs
 
 int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-int pick_cfg(int64_t M, int64_t N) {
+int pick_cfg(int64_t M, int64_t N, int64_t Kp, int out_dtype) {
     if (tiles_of(M, N, 256, 256) >= 256) return kCfgBig;
-    return tiles_of(M, N, 128, 128) >= 256 ? kCfgSmall : kCfgNarrow;
+    const int64_t small = tiles_of(M, N, 128, 128);
+    if (small > 512 && (out_dtype == AXS6_F32 || Kp > kBigShortK)) return kCfgBig;
+    return small >= 256 ? kCfgSmall : kCfgNarrow;
 }
 
 // output tile of a configuration
@@ -419,7 +432,7 @@ void cfg_tile(int cfg, int* bm, int* bn) {
 int gemm_split_count(int64_t M, int64_t N, int64_t Kp) {
     if (M <= 0 || N <= 0) return 1;   // nothing to split (and no division by a zero tile count)
     int bm, bn;
-    cfg_tile(pick_cfg(M, N), &bm, &bn);
+    cfg_tile(pick_cfg(M, N, Kp, AXS6_F32), &bm, &bn);   // the output types differ over 64 tiles only
     const int64_t tiles = tiles_of(M, N, bm, bn);
     const int64_t iters = Kp / kGemmK;
     if (tiles >= 64 || iters < 8) return 1;
@@ -497,7 +510,7 @@ bool gemm_streams_output(const GemmArgs& a, bool split) {
     if (split) return false;
     if ((int64_t)a.M * a.N * (a.out_dtype == AXS6_F32 ? 4 : 2) < ((int64_t)4 << 20)) return false;
     int bm, bn;
-    cfg_tile(pick_cfg(a.M, a.N), &bm, &bn);
+    cfg_tile(pick_cfg(a.M, a.N, a.Kp, a.out_dtype), &bm, &bn);
     return !(bm == 256 && tiles_of(a.M, a.N, bm, bn) <= 256);
 }
 
@@ -518,7 +531,7 @@ int gemm_plan(const GemmArgs& a, GemmPlan* p) {
                  split ? (int)AXS6_F32 : a.out_dtype, per, split ? a.M * a.N : 0,
                  gemm_streams_output(a, split) ? 1 : 0};
     p->splits = splits;
-    const int cfg = pick_cfg(a.M, a.N);
+    const int cfg = pick_cfg(a.M, a.N, a.Kp, a.out_dtype);
     // a long contraction on the narrow tiles: a third slab in flight
     // (2048 x 768, K 3072: 28.5 -> 21.3 us; at K <= 1024 it costs 3-5%)
     p->variant = cfg == kCfgSmall ? kVarSmall
