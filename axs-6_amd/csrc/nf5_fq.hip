@@ -457,7 +457,14 @@ __device__ __forceinline__ int quant_values(float (&f)[V], uint32_t m, const flo
 // 16-byte vector of V values, a block is G = BS / V neighbouring lanes (DPP
 // amax), and the lane writes its V codes and V signs as one V-byte store.
 // Same arithmetic and dither counters as quantize_kernel.
-template <int DT, int BS, bool STOCH>
+// U vectors of a workgroup's contiguous run are loaded together (U == 1: the
+// next one is loaded while one is processed).  The loads in flight bound it:
+// f32, device us, four or more tensors in turn, one ahead -> U = 2: codes
+// alone 11008 x 4096 54.7 -> 47.9, 32768 x 4096 150.6 -> 130.8 (5.0 -> 6.2
+// TB/s); with the FQ output 78.5 -> 76.9, 2048 x 2048 10.1 -> 8.5.  Four are
+// slower (codes alone 49.4).  16-bit vectors hold twice the work per load and
+// keep U = 1 (8192 x 4096 bf16 with the FQ output 37.7, U = 2 38.9).
+template <int DT, int BS, bool STOCH, int U>
 __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(
     const typename Elem<DT>::S* x, int64_t n_vec, const float* __restrict__ lut_g, const uint8_t* __restrict__ band_g,
     const uint8_t* __restrict__ rev_g, uint64_t seed, const uint64_t* __restrict__ seed_dev, uint64_t offset,
@@ -472,48 +479,64 @@ __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(
     __shared__ uint32_t band_w[kBandSize / 4];
     __shared__ uint8_t rev_s[kLutSize];
     const u32x4* xv = reinterpret_cast<const u32x4*>(x);
-    const int64_t step = (int64_t)gridDim.x * kThreads;
+    const int64_t step = (int64_t)gridDim.x * (U * kThreads);
     // the bound is rounded up to whole waves so every lane of a block's DPP
     // group runs every iteration
     const int64_t span = (n_vec + 63) / 64 * 64;
-    int64_t vi = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    // the first vector's HBM load goes out before the tables are staged (the
-    // two latencies overlap); later ones one iteration ahead
-    u32x4 cur = vi < n_vec ? ld_stream(xv + vi) : u32x4{0u, 0u, 0u, 0u};
+    constexpr bool PF = U == 1;
+    u32x4 cur[U], nxt;
+    auto fetch = [&](int64_t base) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = base + u * kThreads;
+            cur[u] = i < n_vec ? ld_stream(xv + i) : u32x4{0u, 0u, 0u, 0u};
+        }
+    };
+    // the first vectors' HBM loads go out before the tables are staged (the
+    // latencies overlap)
+    int64_t base = (int64_t)blockIdx.x * (U * kThreads) + threadIdx.x;
+    fetch(base);
     reinterpret_cast<uint32_t*>(rev_s)[threadIdx.x] = reinterpret_cast<const uint32_t*>(rev_g)[threadIdx.x];
     stage_tables(lut_s, band_w, lut_g, band_g);
     const uint8_t* band_s = reinterpret_cast<const uint8_t*>(band_w);
-    for (; vi < span; vi += step) {
-        const bool live = vi < n_vec;
-        const u32x4 nxt = vi + step < n_vec ? ld_stream(xv + vi + step) : u32x4{0u, 0u, 0u, 0u};
-        float f[V];
-        E::unpack(cur, f);
-        cur = nxt;
-        uint32_t m = 0;
+    while (base < span) {
+        if constexpr (PF) nxt = base + step < n_vec ? ld_stream(xv + base + step) : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            const uint32_t a = __float_as_uint(f[e]) & 0x7fffffffu;
-            m = m > a ? m : a;
-        }
-        m = group_umax<G>(m);
-        float d[V];
-        const DitherVec dv = dither_vec(key, offset + (uint64_t)(vi * V));
+        for (int u = 0; u < U; ++u) {
+            const int64_t vi = base + u * kThreads;
+            if (vi >= span) return;
+            const bool live = vi < n_vec;
+            float f[V];
+            E::unpack(cur[u], f);
+            uint32_t m = 0;
 #pragma unroll
-        for (int e = 0; e < V; ++e) d[e] = STOCH ? dither_step(dv, e) : 0.0f;
-        uint32_t cw[2], sw[2];                         // V bytes of codes and signs
-        const int ex = quant_values<V, STOCH>(f, m, d, lut_s, band_s, rev_s, fq != nullptr, cw, sw);
-        // the outputs are written once: streaming stores
-        if (live) {
-            if constexpr (V == 4) {
-                st_stream(cw[0], reinterpret_cast<uint32_t*>(codes) + vi);
-                if (signs) st_stream(sw[0], reinterpret_cast<uint32_t*>(signs) + vi);
-            } else {
-                st_stream(u32x2{cw[0], cw[1]}, reinterpret_cast<u32x2*>(codes) + vi);
-                if (signs) st_stream(u32x2{sw[0], sw[1]}, reinterpret_cast<u32x2*>(signs) + vi);
+            for (int e = 0; e < V; ++e) {
+                const uint32_t a = __float_as_uint(f[e]) & 0x7fffffffu;
+                m = m > a ? m : a;
             }
-            if (vi % G == 0) st_stream((uint8_t)ex, exps + vi / G);
+            m = group_umax<G>(m);
+            float d[V];
+            const DitherVec dv = dither_vec(key, offset + (uint64_t)(vi * V));
+#pragma unroll
+            for (int e = 0; e < V; ++e) d[e] = STOCH ? dither_step(dv, e) : 0.0f;
+            uint32_t cw[2], sw[2];                         // V bytes of codes and signs
+            const int ex = quant_values<V, STOCH>(f, m, d, lut_s, band_s, rev_s, fq != nullptr, cw, sw);
+            // the outputs are written once: streaming stores
+            if (live) {
+                if constexpr (V == 4) {
+                    st_stream(cw[0], reinterpret_cast<uint32_t*>(codes) + vi);
+                    if (signs) st_stream(sw[0], reinterpret_cast<uint32_t*>(signs) + vi);
+                } else {
+                    st_stream(u32x2{cw[0], cw[1]}, reinterpret_cast<u32x2*>(codes) + vi);
+                    if (signs) st_stream(u32x2{sw[0], sw[1]}, reinterpret_cast<u32x2*>(signs) + vi);
+                }
+                if (vi % G == 0) st_stream((uint8_t)ex, exps + vi / G);
+            }
+            if (fq && live) st_stream(E::pack(f), reinterpret_cast<u32x4*>(fq) + vi);
         }
-        if (fq && live) st_stream(E::pack(f), reinterpret_cast<u32x4*>(fq) + vi);
+        base += step;
+        if constexpr (PF) cur[0] = nxt;
+        else fetch(base);
     }
 }
 
@@ -587,7 +610,11 @@ __global__ __launch_bounds__(kThreads) void quantize_short_kernel(
 }
 
 // Vector form of dequantize_kernel (cols % bs == 0, 4-byte aligned codes and
-// signs, 16-byte aligned y): four values per lane, one 16-byte store.
+// signs, 16-byte aligned y): four values per lane, one 16-byte store.  A
+// lane's loads are 4 bytes, so the bytes in flight bound it: U groups are
+// loaded together (positions past the end load the last group), kDequantTwoGroups
+// says when.
+template <int U>
 __global__ __launch_bounds__(kThreads) void dequantize_vec_kernel(const uint8_t* __restrict__ exps,
                                                                   const uint8_t* __restrict__ codes,
                                                                   const uint8_t* __restrict__ signs,
@@ -597,20 +624,33 @@ __global__ __launch_bounds__(kThreads) void dequantize_vec_kernel(const uint8_t*
     if (threadIdx.x < kLevels) cb[threadIdx.x] = cb_g[threadIdx.x];
     __syncthreads();
     const int sh = bs == 8 ? 1 : (bs == 16 ? 2 : 3);    // groups of 4 per block: 2^sh
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kThreads) {
-        const uint32_t cw = ld_stream(reinterpret_cast<const uint32_t*>(codes) + i);
-        const uint32_t sw = signs ? ld_stream(reinterpret_cast<const uint32_t*>(signs) + i) : 0u;
-        const float scale = pow2_float((int)exps[i >> sh] - kExpBias);
-        float v[4];
+    for (int64_t base = (int64_t)blockIdx.x * (U * kThreads) + threadIdx.x; base < n4;
+         base += (int64_t)gridDim.x * (U * kThreads)) {
+        uint32_t cw[U], sw[U];
+        int ex[U];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float a = cb[(cw >> (8 * e)) & 31] * scale;
-            v[e] = ((sw >> (8 * e)) & 0xffu) ? -a : a;
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = base + u * kThreads < n4 ? base + u * kThreads : n4 - 1;
+            cw[u] = ld_stream(reinterpret_cast<const uint32_t*>(codes) + i);
+            sw[u] = signs ? ld_stream(reinterpret_cast<const uint32_t*>(signs) + i) : 0u;
+            ex[u] = exps[i >> sh];
         }
-        u32x4 w;
-        w.x = __float_as_uint(v[0]); w.y = __float_as_uint(v[1]);
-        w.z = __float_as_uint(v[2]); w.w = __float_as_uint(v[3]);
-        st_stream(w, reinterpret_cast<u32x4*>(y) + i);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = base + u * kThreads;
+            if (i >= n4) break;
+            const float scale = pow2_float(ex[u] - kExpBias);
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a = cb[(cw[u] >> (8 * e)) & 31] * scale;
+                v[e] = ((sw[u] >> (8 * e)) & 0xffu) ? -a : a;
+            }
+            u32x4 w;
+            w.x = __float_as_uint(v[0]); w.y = __float_as_uint(v[1]);
+            w.z = __float_as_uint(v[2]); w.w = __float_as_uint(v[3]);
+            st_stream(w, reinterpret_cast<u32x4*>(y) + i);
+        }
     }
 }
 
@@ -965,6 +1005,18 @@ void launch_fq(const void* x, void* y, int64_t rows, int64_t cols, int bs, bool 
     else launch_fq_typed<DT, 32>(x, y, rows, cols, stochastic, seed, seed_dev, offset, t, st);
 }
 
+// f32 vectors from which quantize_vec_kernel without an FQ output makes two
+// iterations per workgroup, which halves the table staging; us, one -> two:
+// 4096 x 2048 12.4 -> 11.8, 4096 x 4096 22.8 -> 20.2, 8192 x 4096 40.6 -> 36.8;
+// 2048 x 2048 7.3 -> 8.0 (too few workgroups then).  With an FQ output one is
+// faster or equal up to 8192 x 4096 (2048 x 2048 8.5 against 10.6).
+constexpr int64_t kQuantTwiceVecs = (int64_t)2 << 20;
+// Groups of four from which dequantize_vec_kernel loads two per lane; us, one ->
+// two: 11008 x 4096 54.3 -> 44.4 (5.0 -> 6.1 TB/s), 4096 x 2048 12.4 -> 11.1, 1448 x
+// 1024 3.8 -> 3.5; 1024 x 1024 3.1 -> 3.3 (four workgroups per CU become two).
+// Four groups per lane: 45.6 at 11008 x 4096.
+constexpr int64_t kDequantTwoGroups = (int64_t)5 << 16;
+
 template <int DT, int BS>
 void launch_quant_typed(const void* x, int64_t rows, int64_t cols, bool stochastic, uint64_t seed, const uint64_t* seed_dev,
                         uint64_t offset, uint8_t* exps, uint8_t* codes, uint8_t* signs, void* fq,
@@ -974,11 +1026,13 @@ void launch_quant_typed(const void* x, int64_t rows, int64_t cols, bool stochast
     if (cols % BS == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)codes % V == 0 && (uintptr_t)signs % V == 0 &&
         (uintptr_t)fq % 16 == 0) {
         const int64_t n_vec = rows * cols / V;
-        const dim3 grid((unsigned)capped_grid(n_vec, (int64_t)kThreads * 2));   // two iterations per workgroup
+        constexpr int U = DT == AXS6_F32 ? 2 : 1;
+        const int per = U == 1 || (!fq && n_vec >= kQuantTwiceVecs) ? 2 : 1;   // iterations per workgroup
+        const dim3 grid((unsigned)capped_grid(n_vec, (int64_t)kThreads * U * per));
         if (stochastic)
-            quantize_vec_kernel<DT, BS, true><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
+            quantize_vec_kernel<DT, BS, true, U><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
         else
-            quantize_vec_kernel<DT, BS, false><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
+            quantize_vec_kernel<DT, BS, false, U><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
         return;
     }
     const int64_t nblk = (cols + BS - 1) / BS;
@@ -1102,7 +1156,9 @@ extern "C" int axs6_nf5_dequantize(const uint8_t* exponents, const uint8_t* code
     const int64_t nblk = (cols + block_size - 1) / block_size;
     if (cols % block_size == 0 && (uintptr_t)codes % 4 == 0 && (uintptr_t)signs % 4 == 0 && (uintptr_t)y % 16 == 0) {
         const int64_t n4 = rows * cols / 4;
-        dequantize_vec_kernel<<<dim3((unsigned)capped_grid(n4, kThreads)), kThreads, 0, (hipStream_t)stream>>>(
+        const bool two = n4 >= kDequantTwoGroups;
+        const dim3 grid((unsigned)capped_grid(n4, (int64_t)kThreads * (two ? 2 : 1)));
+        (two ? dequantize_vec_kernel<2> : dequantize_vec_kernel<1>)<<<grid, kThreads, 0, (hipStream_t)stream>>>(
             exponents, codes, signs, y, n4, block_size, t.codebook);
         return check_launch(fn);
     }

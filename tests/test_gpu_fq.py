@@ -287,6 +287,28 @@ def test_dequantize_vs_oracle(bs, cols):
     assert bits_equal(dequantize_unified(q).cpu().numpy(), g[f"deq_bs{bs}"])
 
 
+# Whole blocks in runs of two vectors per lane: less than a wave, a run cut in
+# its second half, the first size that dequantizes two groups per lane (and not
+# a multiple of its run), the first that quantizes two runs per workgroup.
+@pytest.mark.parametrize("shape", [(3, 8), (129, 24), (1281, 1032), (8201, 1032)], ids=str)
+def test_codec_vector_runs(shape):
+    from axs.unified.quantize_unified import dequantize_unified, quantize_unified
+
+    x = config2_input(shape, 83)
+    q = quantize_unified(x.to(DEV), 8)
+    oe, oc, os_ = oracle.quantize(x.numpy(), 8)
+    assert np.array_equal(q.shared_exponents.cpu().numpy().reshape(oe.shape), oe)
+    assert np.array_equal(q.magnitudes.cpu().numpy().reshape(oc.shape), oc)
+    d = dequantize_unified(q).cpu().numpy()
+    want = oracle.dequantize(oe, oc, os_, x.shape[1], 8)
+    assert bits_equal(d, want), first_mismatch(d, want)
+    e, c, s, fq = _quant(x.to(DEV), 8, "stochastic", 5)
+    u = oracle.uniform(5, 0, x.numel())
+    oe, oc, os_ = oracle.quantize(x.numpy(), 8, u)
+    assert np.array_equal(c.reshape(oc.shape), oc) and np.array_equal(s.reshape(os_.shape), os_)
+    assert bits_equal(fq, oracle.fake_quantize(x.numpy(), 8, u))
+
+
 # Row-segment kernel (fq_rows_kernel): rows of >= 64 values that do not tile
 # into 16-byte vectors of whole blocks -- a ragged last block, or a view whose
 # start is off 16-byte alignment.  One segment per wave (64 columns), four
