@@ -266,8 +266,12 @@ __global__ __launch_bounds__(NT * RPW) void pack_rows_kernel(PackRowsK k, PackRo
                 if (vi < nvec) {
                     if constexpr (DEFER) {
                         // e1v[j] <= row max, so 2^(e1 - S_row) <= 2^15: finite; below 2^-149 it is 0,
-                        // as is the fp16 value of anything that small
-                        if (e1v[j] != INT_MIN) store_f16_mul<V>(orow + vi * V, f[j], __builtin_amdgcn_ldexpf(1.0f, e1v[j] - S_row));
+                        // as is the fp16 value of anything that small.  A zero block's e1 is 0,
+                        // past the maximum of a row under 2^0: held there, or 0 * inf would be NaN
+                        const int sh = e1v[j] - S_row;
+                        if (e1v[j] != INT_MIN)
+                            store_f16_mul<V>(orow + vi * V, f[j],
+                                             __builtin_amdgcn_ldexpf(1.0f, sh < kF16MaxExp ? sh : kF16MaxExp));
                         else store_f16<V>(orow + vi * V, f[j], -S_row, nullptr);
                     } else {
                         store_f16<V>(orow + vi * V, f[j], -S_row, COLX ? cx[j] : nullptr);

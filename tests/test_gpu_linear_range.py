@@ -182,3 +182,27 @@ def test_nan_and_inf_propagate_like_the_fp32_product(path):
     fin = np.isfinite(want)
     assert fin.sum() > 0.8 * fin.size
     assert oracle.rel_l2(got[fin], want[fin]) < (1e-3 if path == "packed" else 1e-5)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16], ids=str)
+def test_forward_zero_blocks_in_tiny_rows(dt):
+    """Zero blocks in a row whose largest block lies under 2^-113: the row's
+    shift is past 2^128 from a zero block's own exponent, 0.  Whole waves of them:
+    a wave with a tiny block takes the general sequence."""
+    from axs.unified import hip_linear
+
+    M, N, K = 40, 96, 2048
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(M, K, generator=g)
+    w = torch.randn(N, K, generator=g)
+    x[:, 32:64] = 0.0
+    w[:, 1024:] = 0.0
+    x, w = (x * 2.0 ** 100).to(dt), (w * 2.0 ** -120).to(dt)
+    for a, b in ((x, w), (w, x)):     # either operand the tiny one
+        y, _ = hip_linear.forward_train(a.to(DEV), b.to(DEV), None, BS, True)
+        aq = oracle.fake_quantize(a.float().numpy(), BS)
+        bq = oracle.fake_quantize(b.float().numpy(), BS)
+        want = torch.from_numpy(aq).to(dt).double() @ torch.from_numpy(bq).to(dt).double().t()
+        assert bool(torch.isfinite(y).all())
+        # both operands' 11-bit rounding (3.2e-4 measured on Gaussian rows); bf16: the output's 2^-9
+        assert oracle.rel_l2(y.double().cpu().numpy(), want.numpy()) <= (1e-3 if dt == torch.float32 else 2.0 ** -9)
