@@ -31,6 +31,12 @@
 // operands).  f32 values take 11-bit fp16 magnitudes +-lut with the block's
 // 2^e1 applied to the block's product in f32 -- one 16x16x32 MFMA is one block
 // -- against X packed as in the training forward: the same operand rounding.
+// The sums carry the blocks' own scales while those lie in [2^kRefLow,
+// 2^kRefHigh], where no sum overflows or loses digits whatever X's scale.  A
+// workgroup that meets a block outside runs its range a second time with each
+// row's scales relative to its largest (the training forward packs every row so),
+// and the epilogue puts that exponent back: the loop proper carries no state for
+// it, the blocks outside already leave the short sequence.
 #include "nf5_device.h"
 
 #include "gemm_tile.h"
@@ -48,12 +54,20 @@ constexpr int kBfTab = 1 + 6 * 128;      // bf16 magnitudes in the block's six u
 // f32: block scales are stored as 2^(e1 - 15) and X's rows are packed up to 2^15,
 // so a partial sum is the product's own size, not 2^15 over it
 constexpr int kScaleDown = 15;
+// Block exponents whose products need no reference: a block's product is under
+// 2^20 times its scale 2^(e1 - 15), so a sum of 2^25 blocks under 2^(90 + 5 + 25),
+// and at 2^(-80 - 15) an X value 2^30 under its row's largest still leaves a
+// normal product.  The magnitudes that have them:
+constexpr int kRefLow = -80, kRefHigh = 90;
+constexpr uint32_t kRefLowBits = (uint32_t)(kExpBias + kRefLow - 1) << 23;
+constexpr uint32_t kRefHighBits = (uint32_t)(kExpBias + kRefHigh) << 23;
 constexpr int kOob = 0x7ffffff0;         // a buffer offset past every operand (they stay under 2 GiB)
 
 struct InferK {
     const void* x; int ldx;              // FQ(X) as MFMA operand: fp16 (f32 input) or the 16-bit type
     const void* w; const int32_t* sx;    // sx: X's row shifts (f32 input)
     const void* bias; int bias_dtype; void* out; float* partial;
+    int* again; int* refs;               // f32, K split: a second pass was run [split][tile], its exponents [..][kIN]
     int M, N, K, dtype;
     int steps;                           // K steps per workgroup
     int tiles_n, splits;
@@ -157,7 +171,7 @@ __device__ __forceinline__ void look(const u32x4* raw, const InferTables& t, FqL
         const int e1 = (int)(m >> 23) - 126;
         // the log2 bands are under 256 values wide
         const bool band = (m & 0x7fffffu) > 0x7fff00u;
-        const bool sp = m != 0u && (m < kFastMinAmaxBits || e1 >= 128 || band);
+        const bool sp = m != 0u && (m < kRefLowBits || m >= kRefHighBits || band);
         q.special = __builtin_amdgcn_ballot_w64(sp) != 0;
         q.zeros = __builtin_amdgcn_ballot_w64(__float_as_uint(amn) == 0u) != 0;
         q.e1 = m ? e1 : 0;
@@ -175,7 +189,7 @@ __device__ __forceinline__ u32x4 finish(const u32x4* raw, const FqLook<DT>& q, f
     for (int i = 0; i < 4; ++i) r[i] = q.v[2 * i] | (q.v[2 * i + 1] << 16);
     if constexpr (DT == AXS6_F32) {
         const uint32_t w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
-        *scale = pow2_float(q.e1 - kScaleDown);
+        *scale = __builtin_amdgcn_ldexpf(1.0f, q.e1 - kScaleDown);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             // FQ(+-0) = 0 (its sign is of no consequence to a sum); the two values' signs
@@ -200,8 +214,11 @@ __device__ __forceinline__ u32x4 finish(const u32x4* raw, const FqLook<DT>& q, f
 }
 
 // The same 8 values by the general sequence (a wave whose look was special).
+// f32: the scale is taken down by `down`, and *outside set where the block's
+// exponent lies outside [kRefLow, kRefHigh].
 template <int DT>
-__device__ __forceinline__ u32x4 fq_general(const u32x4* raw, const InferTables& t, float* scale) {
+__device__ __forceinline__ u32x4 fq_general(const u32x4* raw, const InferTables& t, int down, float* scale,
+                                            int* outside) {
     const uint8_t* band_s = reinterpret_cast<const uint8_t*>(t.band);
     float f[8];
     if constexpr (DT == AXS6_F32) {
@@ -222,20 +239,18 @@ __device__ __forceinline__ u32x4 fq_general(const u32x4* raw, const InferTables&
         for (int e = 0; e < 8; ++e) f[e] = fq_value(f[e], s, t.lut, false, 0.0f);
         return Elem<DT>::pack(f);
     } else {
-        // a tiny block keeps its magnitudes and a small scale; NaN and
-        // infinite scales give the operand's NaN and inf themselves
+        // the FQ value (a tiny block's is rounded to f32's subnormals) over 2^e1;
+        // NaN and infinite scales give the operand's NaN and inf themselves
         uint32_t r[4];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const uint32_t ab = __float_as_uint(f[e]) & 0x7fffffffu;
-            uint32_t h = t.mag[lut_index(normalise(ab, s), false, 0.0f)];
-            if (s.nan_block) h = 0x7e00u;
-            else if (s.inf_scale) h = ab ? 0x7c00u : 0x7e00u;
-            else if (!ab) h = 0u;
-            h |= (__float_as_uint(f[e]) >> 16) & 0x8000u;
+            const float v = fq_value(f[e], s, t.lut, false, 0.0f);
+            const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)__builtin_amdgcn_ldexpf(v, -s.e1));
             r[e >> 1] = e & 1 ? r[e >> 1] | (h << 16) : h;
         }
-        *scale = (s.nan_block || s.inf_scale) ? 1.0f : __builtin_amdgcn_ldexpf(1.0f, s.e1 - kScaleDown);
+        const bool nonfinite = s.nan_block || s.inf_scale;
+        *scale = nonfinite ? 1.0f : __builtin_amdgcn_ldexpf(1.0f, s.e1 - down);
+        if (!nonfinite && !s.zero && (s.e1 < kRefLow || s.e1 > kRefHigh)) *outside = 1;
         u32x4 out;
         out.x = r[0]; out.y = r[1]; out.z = r[2]; out.w = r[3];
         return out;
@@ -266,13 +281,23 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
 }
 
+// The exponent that a weight row's scales are taken relative to, from the bits
+// of its largest magnitude: 0 inside the window, else its largest block's (at
+// most 127: a block that scales to inf or NaN is its row's result whatever the
+// others sum to).
+__device__ __forceinline__ int row_ref(uint32_t m) {
+    if (m == 0u || (m >= kRefLowBits && m < kRefHighBits)) return 0;
+    return m >= 0x7f000000u ? 127 : m >= 0x00800000u ? (int)(m >> 23) - 126 : 31 - __clz((int)m) - 148;
+}
+
 // Four consecutive outputs of a row, from column col: 2^sh v + bias.
-__device__ __forceinline__ void finish_store(const InferK& k, int row, int col, int sh, const float (&v)[4]) {
+__device__ __forceinline__ void finish_store(const InferK& k, int row, int col, const int (&sh)[4],
+                                             const float (&v)[4]) {
     if (col >= k.N) return;
     float o[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        o[r] = __builtin_amdgcn_ldexpf(v[r], sh) +
+        o[r] = __builtin_amdgcn_ldexpf(v[r], sh[r]) +
                (k.bias && col + r < k.N ? load_elem(k.bias, k.bias_dtype, col + r) : 0.0f);
     const int es = k.dtype == AXS6_F32 ? 4 : 2;
     store4(k.out, k.N, k.N, k.dtype, row, col, o, k.N % 4 == 0 && (uintptr_t)k.out % (4 * es) == 0);
@@ -319,7 +344,8 @@ struct InferTile {
     // The tile's values, finished to the output or (K split) as they lie in the
     // registers: one contiguous KiB per store.  Partial tiles written by rows (64
     // bytes of 16 rows per store) made this 8 us of 256 x 4096 x 11008.
-    __device__ __forceinline__ void store(const InferK& k, int n0, float* part, int fr, int fq) const {
+    // ref: the rows' exponents after a second pass, else null.
+    __device__ __forceinline__ void store(const InferK& k, int n0, float* part, const int* ref, int fr, int fq) const {
         constexpr bool SCALED = DT == AXS6_F32;
         if (k.splits > 1) {
 #pragma unroll
@@ -332,10 +358,15 @@ struct InferTile {
         for (int i = 0; i < TM; ++i) {
             const int row = m + i * 16 + fr;
             if (row >= k.M) continue;
-            const int sh = SCALED ? kScaleDown + k.sx[row] : 0;
+            const int sx = SCALED ? kScaleDown + k.sx[row] : 0;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const float v[4] = {acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]};
+                int sh[4] = {sx, sx, sx, sx};
+                if (SCALED && ref) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sh[r] += ref[n + j * 16 + 4 * fq + r];
+                }
                 finish_store(k, row, n0 + n + j * 16 + 4 * fq, sh, v);
             }
         }
@@ -358,11 +389,38 @@ __global__ __launch_bounds__(256) void infer_reduce_kernel(InferK k) {
     const float* p = k.partial + (int64_t)tile * (BM * kIN) +
                      ((wave * TN + jb % TN) * TM + ib % TM) * 256 + (cq * 16 + r) * 4;
     const int64_t stride = (int64_t)k.tiles_n * (BM * kIN);
-    f32x4m v = *reinterpret_cast<const f32x4m*>(p);
+    const int sx = k.sx ? k.sx[row] + kScaleDown : 0;
+    int sh[4] = {sx, sx, sx, sx};
+    int again = 0;
+    f32x4m v = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 4
-    for (int z = 1; z < k.splits; ++z) v += *reinterpret_cast<const f32x4m*>(p + z * stride);
+    for (int z = 0; z < k.splits; ++z) {
+        v += *reinterpret_cast<const f32x4m*>(p + z * stride);
+        if (k.again) again |= k.again[z * k.tiles_n + tile];
+    }
+    if (again != 0) {
+        // parts with exponents of their own: summed relative to the largest of
+        // those of parts that are not 0
+        int ref[4], top[4] = {INT_MIN, INT_MIN, INT_MIN, INT_MIN};
+        v = f32x4m{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int pass = 0; pass < 2; ++pass) {
+            for (int z = 0; z < k.splits; ++z) {
+                const f32x4m pz = *reinterpret_cast<const f32x4m*>(p + z * stride);
+                const bool own = k.again[z * k.tiles_n + tile] != 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    ref[r] = own ? k.refs[(z * k.tiles_n + tile) * kIN + jb * 16 + 4 * cq + r] : 0;
+                    if (pz[r] == 0.0f) continue;
+                    if (pass == 0) top[r] = ref[r] > top[r] ? ref[r] : top[r];
+                    else v[r] += __builtin_amdgcn_ldexpf(pz[r], ref[r] - top[r]);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sh[r] += top[r] == INT_MIN ? 0 : top[r];
+    }
     const float f[4] = {v[0], v[1], v[2], v[3]};
-    finish_store(k, row, col, k.sx ? k.sx[row] + kScaleDown : 0, f);
+    finish_store(k, row, col, sh, f);
 }
 
 // MW x NW waves over the BM x 128 tile.
@@ -381,6 +439,7 @@ __global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm
     constexpr int D = 2;                             // K steps of raw weight values in flight
     extern __shared__ __align__(16) char smem[];
     __shared__ InferTables tab;
+    __shared__ int ref_s[SCALED ? kIN : 1], again_s;   // f32: the second pass' row exponents; that one is needed
     char* const xs = smem;
     char* const wsl = smem + kXSlabs * XSLAB;
     float* const scl = reinterpret_cast<float*>(wsl + 2 * WSLAB);   // [slab][block][row]
@@ -459,7 +518,7 @@ __global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int row = wrow + 64 * c;
-            if (q[c].special) val[c] = fq_general<DT>(o[c], tab, &scale[c]);
+            if (q[c].special) val[c] = fq_general<DT>(o[c], tab, kScaleDown, &scale[c], &again_s);
             *reinterpret_cast<u32x4*>(slab + swz<kIK>(row, wchunk)) = val[c];
             if constexpr (SCALED) {
                 if ((wchunk & 3) == 0) scl[((s & 1) * 2 + (wchunk >> 2)) * kIN + row] = scale[c];
@@ -485,6 +544,7 @@ __global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm
         }
     }
     if (tid < kBandSize / 4) tab.band[tid] = bandv;
+    if (SCALED && tid == 0) again_s = 0;
     lds_barrier();
     if constexpr (DT == AXS6_BF16) {
         build_bf16_table(tab.mag, tab.lut, tid);
@@ -499,13 +559,7 @@ __global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm
     for (int s = 0;; s += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            if (s + d >= T) {
-                t.store(k, n0,
-                        k.partial + (int64_t)(split * k.tiles_n + tile) * (BM * kIN) + wave * (TM * TN * 256) +
-                            lane * 4,
-                        fr, fq);
-                return;
-            }
+            if (s + d >= T) goto summed;
             // slab s + d has landed once only the W issues after it, and the
             // slab between them, are outstanding
             wait_vmcnt<XI + 2 * WI>();
@@ -523,6 +577,61 @@ __global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm
             store_w(s + d + 1, raw[(d + 1) % D]);
         }
     }
+summed:
+    // the thread's place again: kept across the loop it costs the f32 32-row
+    // instance, at its register limit, a spill
+    const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), et = wave * 64 + el;
+    const int efr = el & 15, efq = el >> 4;
+    bool again = false;
+    if constexpr (SCALED) {
+        lds_barrier();
+        again = __builtin_amdgcn_readfirstlane(again_s) != 0;
+        if (again) {
+            // the largest magnitude of each row's range (a row is 8 lanes' chunks)
+            uint32_t top[2] = {0u, 0u};
+            for (int s = 0; s < T; ++s) {
+                issue_w(s, raw[0]);
+#pragma unroll
+                for (int i = 0; i < 8 * RV; ++i) {
+                    const uint32_t ab = raw[0][i / (4 * RV)][i / 4 % RV][i % 4] & 0x7fffffffu;
+                    uint32_t& m = top[i / (4 * RV)];
+                    m = m > ab ? m : ab;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int ref = row_ref(group_umax<8>(top[c]));
+                if (et % 8 == 0) ref_s[et / 8 + 64 * c] = ref;
+            }
+            t.clear();
+            for (int s = 0; s < T; ++s) {
+                // nothing in flight into the slabs, nobody still reading them
+                wait_vmcnt<0>();
+                lds_barrier();
+                issue_x(s);
+                issue_w(s, raw[0]);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int row = et / 8 + 64 * c, chunk = et % 8;
+                    const u32x4 v = fq_general<DT>(raw[0][c], tab, kScaleDown + ref_s[row], &scale[c], &again_s);
+                    *reinterpret_cast<u32x4*>(wsl + swz<kIK>(row, chunk)) = v;
+                    if (chunk % 4 == 0) scl[chunk / 4 * kIN + row] = scale[c];
+                }
+                wait_vmcnt<0>();
+                lds_barrier();
+                t.multiply(xs + (s % kXSlabs) * XSLAB, wsl, scl, 0, efr, efq);
+                t.multiply(xs + (s % kXSlabs) * XSLAB, wsl, scl, 1, efr, efq);
+            }
+        }
+        if (k.splits > 1) {
+            const int part = split * k.tiles_n + tile;
+            if (et == 0) k.again[part] = again ? 1 : 0;
+            if (again && et < kIN) k.refs[part * kIN + et] = ref_s[et];
+        }
+    }
+    t.store(k, n0,
+            k.partial + (int64_t)(split * k.tiles_n + tile) * (BM * kIN) + wave * (TM * TN * 256) + el * 4,
+            again ? ref_s : nullptr, efr, efq);
 #endif
 }
 
@@ -553,7 +662,7 @@ int run_infer_dt(const InferK& k, int bm, hipStream_t st) {
 }
 
 // Row tile, K split and workspace of a shape.
-struct InferPlan { int bm, steps, splits; size_t xq, sx, partial, total; };
+struct InferPlan { int bm, steps, splits; size_t xq, sx, again, refs, partial, total; };
 
 // Where this form is the faster one.  The packed path's cost is the weight's
 // (a read, a write and a read back), this one's grows with the rows: the FQ of
@@ -596,6 +705,9 @@ bool infer_plan(int64_t M, int64_t N, int64_t K, int dtype, InferPlan* p) {
     const int64_t Kp = pad_to(K, kGemmK);
     p->xq = take((size_t)M * (dtype == AXS6_F32 ? Kp : K) * 2);
     p->sx = take((size_t)M * sizeof(int32_t));
+    const size_t parts = f32 && p->splits > 1 ? (size_t)p->splits * tiles : 0;
+    p->again = parts ? take(parts * sizeof(int)) : 0;
+    p->refs = parts ? take(parts * kIN * sizeof(int)) : 0;
     p->partial = p->splits > 1 ? take((size_t)p->splits * tiles * p->bm * kIN * sizeof(float)) : 0;
     p->total = off;
     return true;
@@ -656,6 +768,10 @@ extern "C" int axs6_nf5_linear_infer(const void* x, const void* w, const void* b
         const int64_t Kp = pad_to(K, kGemmK);
         k.ldx = (int)Kp;
         k.sx = (const int32_t*)(ws + p.sx);
+        if (p.splits > 1) {
+            k.again = (int*)(ws + p.again);
+            k.refs = (int*)(ws + p.refs);
+        }
         const PackRowsArgs px{x, dtype, M, K, 32, qx, false, 0, 0, nullptr, nullptr, (_Float16*)(ws + p.xq), Kp, Kp,
                               (int32_t*)(ws + p.sx), nullptr, nullptr, nullptr};
         rc = launch_pack_rows(px, t, st);

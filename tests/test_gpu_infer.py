@@ -152,3 +152,49 @@ def test_infer_in_graph_replays(m):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, eager), i
+
+
+# f32 weights whose block scales leave the window in which the GEMM form sums
+# without a reference exponent: near the type's top under small inputs, in its
+# subnormals under large ones, and rows that cross it inside the contraction
+# (over the splits of K and inside one).  K split over workgroups and (the last) not.
+@pytest.mark.parametrize("m,K,N", [(5, 1024, 4160), (33, 2080, 2051), (100, 1024, 8200), (5, 1024, 65540)])
+def test_infer_gemm_weight_range(m, K, N):
+    from axs.unified import hip_linear
+
+    print(f"[infer range m={m} K={K} N={N}]", flush=True)
+    assert _form(m, K, N, torch.float32)
+    g = torch.Generator().manual_seed(K + N + m)
+    x = torch.randn(m, K, generator=g)
+    w = torch.randn(N, K, generator=g).clamp_(-4.0, 4.0)   # 4 x 3e37: no block scales to inf
+    w[:, :32].abs_()
+    h = K // 2
+    for xs, ws in ((1e-3, 3e37), (1e-6, 3e37), (1e10, 1e-43), (1e10, 1e-36), (1.0, 1.0)):
+        xv, wv = x * xs, w * ws
+        if ws == 1.0:   # rows of other scales in a tile of ordinary ones
+            wv[1] *= 2.0 ** 112
+            wv[2] *= 2.0 ** -138
+            wv[3, :h] = 0.0          # nothing, then tiny
+            wv[3, h:] *= 2.0 ** -135
+            wv[4, :h] *= 2.0 ** -120   # tiny, then huge
+            wv[4, h:] *= 2.0 ** 112
+            wv[5, h:] *= 2.0 ** -100   # ordinary, then tiny
+            wv[6] = 0.0
+            wv[7, 32:] *= 2.0 ** -140  # one ordinary block
+            xv[:, 64:96] = 0.0
+        y = _infer(xv, wv, None).cpu().double()
+        # the training forward packs every row relative to its largest block
+        # from the same operand values: only the summation orders differ
+        t = hip_linear.forward_train(xv.to(DEV), wv.to(DEV), None)[0].cpu().double()
+        assert bool(torch.isfinite(y).all()), (xs, ws, int((~torch.isfinite(y)).sum()))
+        scale = t.norm(dim=0).clamp_min(1e-300)
+        err = ((y - t).norm(dim=0) / scale).amax()
+        assert err <= 1e-5, (xs, ws, float(err), int(((y - t).norm(dim=0) / scale).argmax()))
+        if ws > 1e-38:   # FQ values of subnormal blocks are rounded once more in the oracle
+            n = 64
+            want = _exact(xv, wv[:n], None)
+            err = ((y[:, :n] - want).norm(dim=0) / want.norm(dim=0).clamp_min(1e-300))
+            ok = torch.ones(n, dtype=torch.bool)
+            if ws == 1.0:
+                ok[[2, 3, 6]] = False
+            assert float(err[ok].amax()) <= 2 * BAR[torch.float32], (xs, ws)
