@@ -64,6 +64,7 @@ struct FusedK {
     int M; int N; int K;
     const float* lut; const uint8_t* band;
     int bias_dtype = AXS6_F32;
+    const float* codebook = nullptr; const uint8_t* rev = nullptr;   // RND f16
 };
 
 // The 8 values lane (row r, group q) takes of a row's 32-block: in bf16/f16
@@ -461,8 +462,12 @@ __device__ __forceinline__ float dec_wave_sum(float v) {
 // contracts them (axs6_nf5_linear_infer); the fused linear proper keeps them in
 // f32.  The table is staged rounded: rounding commutes with 2^e1 while the
 // value is normal in the type, which bf16 shares with f32; f16 blocks outside
-// e1 in [-6, 15] (lut[0] 2^e1 subnormal, or 2^e1 past its range) take the
-// general sequence and are rounded once more there.
+// e1 in [-6, 15] (lut[0] 2^e1 subnormal, or 2^e1 past its range) and blocks
+// the short sequence does not cover take the general one on the unrounded table
+// and are rounded once: f16, whose small weights live there, from the 32 levels
+// and the index's code in LDS (1.1 KiB; the whole table would cost the fourth
+// workgroup of a CU where FQ(X) takes 32 KiB: 2 x 4096 x 11008 25.9 -> 27.3 us);
+// bf16, whose such blocks are all under 2^-100, from memory.
 template <int DT, int MR, int KS, bool QX, bool RND>
 __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) {
     static_assert(!RND || DT != AXS6_F32, "f32 values need no rounding");
@@ -472,11 +477,21 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
     constexpr int NB = kDecPf + 1;
     constexpr int ES = sizeof(S);
     static_assert(kDecWaves % KS == 0, "waves per row");
+    constexpr bool CODES = RND && DT == AXS6_F16;
     __shared__ float lut_s[kLutSize];
+    __shared__ float cb_s[CODES ? kLevels : 1];
+    __shared__ uint32_t rev_w[CODES ? kLutSize / 4 : 1];
     __shared__ uint32_t band_w[kBandSize / 4];
     __shared__ float part_s[kDecWaves * MR];
     extern __shared__ __align__(16) float xq_s[];   // FQ(X) in the lanes' read order
     const uint8_t* band_s = reinterpret_cast<const uint8_t*>(band_w);
+    // fq_value on the unrounded table
+    auto fq_full = [&](float x, const FqScale& s) {
+        if constexpr (!RND) return fq_value(x, s, lut_s, false, 0.0f);
+        const int i = lut_index(normalise(__float_as_uint(x) & 0x7fffffffu, s), false, 0.0f);
+        const float rec = CODES ? cb_s[reinterpret_cast<const uint8_t*>(rev_w)[i]] : k.lut[i];
+        return s.nan_block ? __uint_as_float(kNanBits) : torch_sign(x) * rec * scale_of(s);
+    };
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int SP = (k.K + kDecStep - 1) / kDecStep;       // steps per row
@@ -496,6 +511,10 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
     uint32_t bandv = 0;
     if (tid < kLutSize / 4) lutv = reinterpret_cast<const float4*>(k.lut)[tid];
     if (tid < kBandSize / 4) bandv = reinterpret_cast<const uint32_t*>(k.band)[tid];
+    float cbv = 0.0f;
+    uint32_t revv = 0;
+    if (CODES && tid < kLevels) cbv = k.codebook[tid];
+    if (CODES && tid < kLutSize / 4) revv = reinterpret_cast<const uint32_t*>(k.rev)[tid];
     // X chunk c: row m, step j, lane slot l -> x[m, 512 j + 8 l .. + 7],
     // stored as float4 ((m SP + j) 2 + h) 64 + l (h: first / second four)
     const S* xs = reinterpret_cast<const S*>(k.x);
@@ -528,6 +547,8 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
     }
     if (tid < kLutSize / 4) reinterpret_cast<float4*>(lut_s)[tid] = lutv;
     if (tid < kBandSize / 4) band_w[tid] = bandv;
+    if (CODES && tid < kLevels) cb_s[tid] = cbv;
+    if (CODES && tid < kLutSize / 4) rev_w[tid] = revv;
     __syncthreads();
     auto x_stage = [&](int c, const u32x4 (&v)[L], bool valid) {
         float f[8];
@@ -543,8 +564,13 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
             }
             mx = group_umax<4>(mx);
             const FqScale s = fq_scale(mx, band_s);
-            const float d[8] = {};
-            fq_vector<8>(f, s, lut_s, false, d);
+            if (RND && __builtin_amdgcn_ballot_w64(s.e1 < kFastMinE1 || (CODES && s.e1 < -6)) != 0) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] = fq_full(f[e], s);
+            } else {
+                const float d[8] = {};
+                fq_vector<8>(f, s, lut_s, false, d);
+            }
             if constexpr (RND) round_to_elem<DT, 8>(f);
         }
         if (c < nchunk) {
@@ -586,7 +612,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void fused_decode_kernel(FusedK k) 
         if (__builtin_amdgcn_ballot_w64(wide) != 0) {
             const FqScale s = fq_scale_general(mx, band_s);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] = fq_value(f[e], s, lut_s, false, 0.0f);
+            for (int e = 0; e < 8; ++e) f[e] = fq_full(f[e], s);
             if constexpr (RND) round_to_elem<DT, 8>(f);
             e1 = 0;
         } else {
@@ -885,7 +911,7 @@ bool infer_rows_fit(int64_t M, int64_t N, int64_t K) {
 
 int launch_infer_rows(const void* x, const void* w, const void* bias, int bias_dtype, void* y, int dtype, int64_t M,
                       int64_t N, int64_t K, bool qx, const DeviceTables& t, hipStream_t st) {
-    const FusedK k{x, w, bias, y, (int)M, (int)N, (int)K, t.lut, t.band, bias_dtype};
+    const FusedK k{x, w, bias, y, (int)M, (int)N, (int)K, t.lut, t.band, bias_dtype, t.codebook, t.rev};
     if (dtype == AXS6_F32) launch_decode_rows<AXS6_F32, false>(k, qx, st);
     else if (dtype == AXS6_BF16) launch_decode_rows<AXS6_BF16, true>(k, qx, st);
     else launch_decode_rows<AXS6_F16, true>(k, qx, st);

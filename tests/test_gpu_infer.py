@@ -198,3 +198,41 @@ def test_infer_gemm_weight_range(m, K, N):
             if ws == 1.0:
                 ok[[2, 3, 6]] = False
             assert float(err[ok].amax()) <= 2 * BAR[torch.float32], (xs, ws)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("m", [1, 2, 40])
+def test_infer_subnormal_values_round_once(m, dt):
+    """FQ values that are subnormal in the operands' type, rounded to it once
+    from the table's own value: one product per output, so every bit is defined
+    (the f32 product of the rounded values, rounded to the type)."""
+    from axs.unified import functional_unified as fu
+
+    K, N = 1024, 4160
+    assert _form(m, K, N, dt)
+    lo = -24 if dt == torch.float16 else -133        # the type's smallest power of two
+    top = 0 if dt == torch.float16 else -110
+    g = torch.Generator().manual_seed(21)
+    w = torch.randn(N, K, generator=g) * torch.exp2(torch.randint(lo + 4, top, (N, 1), generator=g).float())
+    w = w.to(dt)
+    one = 1.0 if dt == torch.float16 else 2.0 ** 60
+    x = torch.zeros(m, K)
+    for i in range(m):
+        x[i, 25 * i + 5] = one
+    x = x.to(dt)
+    with torch.no_grad():
+        y = fu.axs_linear_unified(x.to(DEV), w.to(DEV), None, 32, False).cpu()
+    wq = torch.from_numpy(oracle.fake_quantize(w.float().numpy(), 32)).to(dt)
+    pick = x.float().argmax(1)
+    assert torch.equal(y, (wq[:, pick].t().double() * one).to(dt))
+    # the same values as the input, one weight per output row
+    v = w[:m]
+    d = torch.zeros(N, K)
+    d[torch.arange(N), torch.arange(N) % K] = one
+    d = d.to(dt)
+    y = _infer(v, d, None).cpu()
+    vq = torch.from_numpy(oracle.fake_quantize(v.float().numpy(), 32)).to(dt)
+    dq = torch.from_numpy(oracle.fake_quantize(d.float().numpy(), 32)).to(dt)
+    k = torch.arange(N) % K
+    want = (vq[:, k].float() * dq[torch.arange(N), k].float()).to(dt)
+    assert torch.equal(y, want)
