@@ -54,6 +54,9 @@ _SIGNATURES: dict[str, list] = {
     "axs6_nf5_fused_linear_split": [_vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i32, _i32, _vp],
     "axs6_nf5_linear_infer_workspace": [_i64, _i64, _i64, _i32, _i32],
     "axs6_nf5_linear_infer": [_vp, _vp, _vp, _i32, _vp, _i32, _i64, _i64, _i64, _i32, _i32, _vp, _i64, _vp],
+    "axs6_nf5_linear_infer_stacked_workspace": [_i64, _i64, _i64, _i64, _i32, _i32],
+    "axs6_nf5_linear_infer_stacked": [_vp, _vp, _vp, _i32, _vp, _i32, _i64, _i64, _i64, _i64, _i32, _i32, _vp, _i64,
+                                      _vp],
     "axs6_nf5_wire_bytes": [_i64, _i64, _i32],
     "axs6_nf5_pack_wire": [_vp, _i32, _i64, _i64, _i32, _vp, _vp],
     "axs6_nf5_unpack_wire": [_vp, _i64, _i64, _i32, _vp, _vp],
@@ -80,6 +83,7 @@ _RESTYPES = {"axs6_linear_padded_k": _i64, "axs6_nf5_linear_backward_workspace":
              "axs6_nf5_wire_bytes": _i64, "axs6_nf5_block_bytes": _i64, "axs6_multi_tensor_workspace": _i64,
              "axs6_nf5_row_stats_workspace": _i64, "axs6_nf5_fused_linear_split_x": ctypes.c_int32,
              "axs6_nf5_fused_linear_split_workspace": _i64, "axs6_nf5_linear_infer_workspace": _i64,
+             "axs6_nf5_linear_infer_stacked_workspace": _i64,
              "axs6_layer_norm_backward_workspace": _i64}
 
 

@@ -107,8 +107,11 @@ def axs_linear_group_unified(
     as one: the weights stacked along the output dim, so the input is packed
     once and forward and backward each run one linear (one GEMM per
     direction instead of one per weight).  Each output equals its own
-    ``axs_linear_unified`` forward bit for bit (same operand rows, same
-    contraction order); in the backward the input gradient is the contraction
+    ``axs_linear_unified`` forward bit for bit: the packed operands' rows and
+    contraction order do not depend on the other weights, and projections
+    that without a gradient take an inference form, whose order of summation
+    follows the weight's size, keep the order of their own or run one by one.
+    In the backward the input gradient is the contraction
     over all stacked outputs at once, and the stochastic rounding of the
     output gradient draws one stream for the stacked rows (both within the
     linear's tolerance).  This function is this library's; the reference runs
@@ -122,13 +125,20 @@ def axs_linear_group_unified(
     if len(weights) == 1:
         return (axs_linear_unified(input, weights[0], biases[0], block_size, quantize_input, quantize_grad),)
     sizes = [w.shape[0] for w in weights]
+    part_n = hip_linear.group_part_n(input, weights, biases, block_size)
+    if part_n is None:
+        for b, n in zip(biases, sizes):
+            if b is not None and b.shape != (n,):
+                raise RuntimeError(f"axs_linear_group_unified: bias of shape {tuple(b.shape)} for {n} outputs")
+        return tuple(axs_linear_unified(input, w, b, block_size, quantize_input, quantize_grad)
+                     for w, b in zip(weights, biases))
     w = torch.cat(weights, 0)
     if all(b is None for b in biases):
         b = None
     else:
         b = torch.cat([bi if bi is not None else torch.zeros(n, dtype=w.dtype, device=w.device)
                        for bi, n in zip(biases, sizes)])
-    y = axs_linear_unified(input, w, b, block_size, quantize_input, quantize_grad)
+    y = hip_linear.linear_autograd(input, w, b, block_size, quantize_input, quantize_grad, part_n)
     return tuple(y.split(sizes, dim=-1))
 
 

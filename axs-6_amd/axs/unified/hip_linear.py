@@ -165,15 +165,51 @@ def backward(grad_output, saved: Saved, block_size: int, quantize_grad: bool,
         bool(need_x), bool(need_w), bool(need_b), seed, saved.x_dtype)
 
 
-def linear_autograd(input, weight, bias, block_size=32, quantize_input=True, quantize_grad=True):
+# Stacked weights smaller than this (values of one) are one call of the inference
+# form, larger ones a call each: the stacking reads and writes every weight.
+# us, three weights stacked / one by one, 64 rows: 2048 x 2048 bf16 39 / 59, f32
+# 52 / 71; 2560 x 2560 60 / 64, 79 / 79; 3072 x 3072 75 / 68, 93 / 81.
+STACK_INFER_BELOW = 1 << 23
+
+
+def group_part_n(input, weights, biases, block_size: int) -> int | None:
+    """How linears of one input that are to have their own forwards' bits run over
+    the stacked weights: -1, as the training forward; n > 0, in the inference form
+    of weights of n rows; None, not at all (one by one)."""
+    train_like = True
+    for w, b in zip(weights, biases):
+        recorded = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (input, w, b))
+        train_like = train_like and (recorded or _infer_workspace(input, w.shape[0], w, block_size) < 0)
+    if train_like:
+        return -1
+    n, K = weights[0].shape
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (input, *weights, *biases)):
+        return None
+    if any(w.shape != weights[0].shape or w.dtype != weights[0].dtype for w in weights) or n * K >= STACK_INFER_BELOW:
+        return None
+    return n if _infer_workspace(input, n * len(weights), weights[0], block_size) >= 0 else None
+
+
+def _infer_workspace(input, N: int, weight, block_size: int) -> int:
+    """The library's workspace query for a linear without gradients of N stacked
+    rows whose weights are like `weight`: -1 where it takes the training forward."""
+    part_n, K = weight.shape
+    rows = input.numel() // K if K else 0
+    dtype = input.dtype if input.dtype in _SUPPORTED else torch.float32
+    return _lib.lib().axs6_nf5_linear_infer_stacked_workspace(rows, N, K, part_n, _lib.DTYPE_CODE[dtype], block_size)
+
+
+def linear_autograd(input, weight, bias, block_size=32, quantize_input=True, quantize_grad=True, part_n=0):
     """``axs_linear_unified`` as one C++ autograd node (axs._C.linear): the
     same forward and backward as forward_train / backward, with no Python on
-    either side of the engine."""
+    either side of the engine.  ``part_n``: the rows of one of the weights
+    stacked in ``weight`` (0: it is one weight; -1: the training forward also
+    where no gradient is recorded)."""
     fn = "axs_linear"
     _require_device(input, fn)
     _require_device(weight, fn)
     assert block_size in VALID_BLOCK_SIZES, f"block_size must be one of {VALID_BLOCK_SIZES}"
-    return _lib.ext().linear(input, weight, bias, block_size, bool(quantize_input), bool(quantize_grad))
+    return _lib.ext().linear(input, weight, bias, block_size, bool(quantize_input), bool(quantize_grad), part_n)
 
 
 def _matmul_2d(a2: torch.Tensor, bt: torch.Tensor, count: int, rows_b: int) -> torch.Tensor:

@@ -681,21 +681,23 @@ struct InferPlan { int bm, steps, splits; size_t xq, sx, again, refs, partial, t
 //    128 x 2048 x 2048         -         26.2 / 27.8
 //    128 x 1024 x 1024    17.3 / 17.4    17.7 / 19.5
 //     16 x 512 x 11008         -         16.6 / 19.2
-bool infer_plan(int64_t M, int64_t N, int64_t K, int dtype, InferPlan* p) {
+// part_n: the rows of one of the weights that make up W, whose plan it takes (N:
+// W is one weight).
+bool infer_plan(int64_t M, int64_t N, int64_t K, int64_t part_n, int dtype, InferPlan* p) {
     const bool f32 = dtype == AXS6_F32;
-    const int64_t most = N * K >= (int64_t)1 << 23 ? (f32 ? 128 : 256) : (f32 ? 64 : 128);
-    if (M < 3 || M > most || K < 1024 || N * K < (int64_t)1 << 22) return false;
+    const int64_t most = part_n * K >= (int64_t)1 << 23 ? (f32 ? 128 : 256) : (f32 ? 64 : 128);
+    if (M < 3 || M > most || K < 1024 || part_n * K < (int64_t)1 << 22) return false;
     // 32-bit buffer offsets
     if (N * K * (f32 ? 4 : 2) >= (int64_t)kOob || M * (K + kGemmK) * 2 >= (int64_t)kOob) return false;
     p->bm = M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256;
-    const int64_t tiles = (N + kIN - 1) / kIN;
+    const int64_t tiles = (N + kIN - 1) / kIN, part_tiles = (part_n + kIN - 1) / kIN;
     const int64_t steps = (K + kIK - 1) / kIK;
     // K splits: rounds of workgroups times the steps of each, the fill of its
     // pipeline (about 4 steps) and the partial sums' traffic (about 1 step per split)
     const int64_t slots = p->bm >= 128 ? 256 : 512;
     int64_t s = 1, best = INT64_MAX;
     for (int64_t c = 1; c <= 16 && c <= steps / 4 + 1; ++c) {
-        const int64_t cost = ((tiles * c + slots - 1) / slots) * (((steps + c - 1) / c) + 4) + (c > 1 ? 2 + c : 0);
+        const int64_t cost = ((part_tiles * c + slots - 1) / slots) * (((steps + c - 1) / c) + 4) + (c > 1 ? 2 + c : 0);
         if (cost < best) { best = cost; s = c; }
     }
     p->steps = (int)((steps + s - 1) / s);
@@ -718,19 +720,33 @@ bool infer_plan(int64_t M, int64_t N, int64_t K, int dtype, InferPlan* p) {
 
 using namespace axs6;
 
+extern "C" int64_t axs6_nf5_linear_infer_stacked_workspace(int64_t M, int64_t N, int64_t K, int64_t part_n,
+                                                           int32_t dtype, int32_t block_size) {
+    if (!valid_dtype(dtype) || block_size != 32 || M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || M > (1 << 30) ||
+        N > (1 << 30) || K > (1 << 30) || part_n <= 0 || part_n > N)
+        return -1;
+    // the streamed form's waves per row follow the weight's size
+    if (infer_rows_fit(M, N, K)) return part_n == N ? 0 : -1;
+    InferPlan p;
+    return infer_plan(M, N, K, part_n, dtype, &p) ? (int64_t)p.total : -1;
+}
+
 extern "C" int64_t axs6_nf5_linear_infer_workspace(int64_t M, int64_t N, int64_t K, int32_t dtype,
                                                    int32_t block_size) {
-    if (!valid_dtype(dtype) || block_size != 32 || M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || M > (1 << 30) ||
-        N > (1 << 30) || K > (1 << 30))
-        return -1;
-    if (infer_rows_fit(M, N, K)) return 0;
-    InferPlan p;
-    return infer_plan(M, N, K, dtype, &p) ? (int64_t)p.total : -1;
+    return axs6_nf5_linear_infer_stacked_workspace(M, N, K, N, dtype, block_size);
 }
 
 extern "C" int axs6_nf5_linear_infer(const void* x, const void* w, const void* bias, int32_t bias_dtype, void* y,
                                      int32_t dtype, int64_t M, int64_t N, int64_t K, int32_t block_size,
                                      int32_t quantize_input, void* workspace, int64_t workspace_bytes, void* stream) {
+    return axs6_nf5_linear_infer_stacked(x, w, bias, bias_dtype, y, dtype, M, N, K, N, block_size, quantize_input,
+                                         workspace, workspace_bytes, stream);
+}
+
+extern "C" int axs6_nf5_linear_infer_stacked(const void* x, const void* w, const void* bias, int32_t bias_dtype,
+                                             void* y, int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t part_n,
+                                             int32_t block_size, int32_t quantize_input, void* workspace,
+                                             int64_t workspace_bytes, void* stream) {
     const char* fn = "axs6_nf5_linear_infer";
     if (!valid_dtype(dtype) || (bias && !valid_dtype(bias_dtype)))
         return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: unknown dtype code %d", fn, valid_dtype(dtype) ? bias_dtype : dtype);
@@ -738,7 +754,7 @@ extern "C" int axs6_nf5_linear_infer(const void* x, const void* w, const void* b
         return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: block_size must be 32 (got %d)", fn, block_size);
     if (M < 0 || N < 0 || K < 0) return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: negative dimension", fn);
     if (M == 0 || N == 0) return AXS6_OK;
-    const int64_t need = axs6_nf5_linear_infer_workspace(M, N, K, dtype, block_size);
+    const int64_t need = axs6_nf5_linear_infer_stacked_workspace(M, N, K, part_n, dtype, block_size);
     if (need < 0) return fail(AXS6_ERR_UNSUPPORTED, "%s: no inference form for this shape (use the forward)", fn);
     if (!x || !w || !y) return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
     if ((uintptr_t)x % 16 || (uintptr_t)w % 16)
@@ -754,7 +770,7 @@ extern "C" int axs6_nf5_linear_infer(const void* x, const void* w, const void* b
     if (infer_rows_fit(M, N, K)) return launch_infer_rows(x, w, bias, bias_dtype, y, dtype, M, N, K, qx, t, st);
 
     InferPlan p;
-    infer_plan(M, N, K, dtype, &p);
+    infer_plan(M, N, K, part_n, dtype, &p);
     char* ws = (char*)workspace;
     InferK k{};
     k.w = w; k.bias = bias; k.bias_dtype = bias_dtype; k.out = y; k.dtype = dtype;

@@ -249,9 +249,10 @@ struct Fwd {
 };
 
 // train = false: no backward will follow, so where the library has an inference
-// form for the shape it runs instead and the packed operands stay undefined.
+// form for the shape it runs instead and the packed operands stay undefined;
+// part_n: the rows of one of the weights stacked in `weight` (0: it is one).
 Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
-                    int64_t bs, bool quantize_input, bool train = true) {
+                    int64_t bs, bool quantize_input, bool train = true, int64_t part_n = 0) {
     const char* fn = "axs_linear";
     require_device(input, fn);
     require_device(weight, fn);
@@ -269,7 +270,9 @@ Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std
     Fwd r;
     if (!train) {
         const int64_t M = x2.size(0);
-        const int64_t ws = axs6_nf5_linear_infer_workspace(M, N, K, dtype_code(dtype), (int32_t)bs);
+        if (part_n <= 0) part_n = N;
+        const int64_t ws =
+            axs6_nf5_linear_infer_stacked_workspace(M, N, K, part_n, dtype_code(dtype), (int32_t)bs);
         if (ws >= 0) {
             at::Tensor w2 = dense(weight.to(dtype)), b;
             if (bias && bias->defined()) {
@@ -279,10 +282,11 @@ Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std
             at::Tensor y = at::empty({M, N}, x2.options());
             at::Tensor work = ws ? at::empty({ws}, x2.options().dtype(at::kByte)) : at::Tensor();
             c10::DeviceGuard guard(x2.device());
-            check_rc(axs6_nf5_linear_infer(x2.data_ptr(), w2.data_ptr(), b.defined() ? b.data_ptr() : nullptr,
-                                           b.defined() ? dtype_code(b.scalar_type()) : AXS6_F32, y.data_ptr(),
-                                           dtype_code(dtype), M, N, K, (int32_t)bs, quantize_input ? 1 : 0,
-                                           ws ? work.data_ptr() : nullptr, ws, stream_of(x2)),
+            check_rc(axs6_nf5_linear_infer_stacked(
+                         x2.data_ptr(), w2.data_ptr(), b.defined() ? b.data_ptr() : nullptr,
+                         b.defined() ? dtype_code(b.scalar_type()) : AXS6_F32, y.data_ptr(), dtype_code(dtype), M, N,
+                         K, part_n, (int32_t)bs, quantize_input ? 1 : 0, ws ? work.data_ptr() : nullptr, ws,
+                         stream_of(x2)),
                      "axs6_nf5_linear_infer");
             r.out = to_input_dtype(y.reshape(lead_shape(input.sizes(), N)), input.scalar_type());
             return r;
@@ -376,9 +380,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> linear_bwd_impl(
 struct LinearFunction : public torch::autograd::Function<LinearFunction> {
     static at::Tensor forward(AutogradContext* ctx, const at::Tensor& input, const at::Tensor& weight,
                               const at::Tensor& bias, int64_t bs, bool quantize_input, bool quantize_grad,
-                              bool has_bias, bool train) {
+                              bool has_bias, bool train, int64_t part_n) {
         Fwd r = linear_fwd_impl(input, weight, has_bias ? std::optional<at::Tensor>(bias) : std::nullopt, bs,
-                                quantize_input, train);
+                                quantize_input, train, part_n);
         if (!train) return r.out;   // nothing records a gradient: nothing to save
         ctx->save_for_backward({r.xq, r.sx, r.wq, r.sw});
         auto& d = ctx->saved_data;
@@ -396,7 +400,7 @@ struct LinearFunction : public torch::autograd::Function<LinearFunction> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const at::Tensor& g = grads[0];
         if (!g.defined())
-            return variable_list(8);
+            return variable_list(9);
         const auto saved = ctx->get_saved_variables();
         auto& d = ctx->saved_data;
         const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
@@ -407,20 +411,22 @@ struct LinearFunction : public torch::autograd::Function<LinearFunction> {
             d["n_true"].toInt(), d["k_true"].toInt(), (at::ScalarType)d["dtype"].toInt(), x_shape,
             (at::ScalarType)d["w_dtype"].toInt(), d["bs"].toInt(), d["quantize_grad"].toBool(), need_x, need_w,
             need_b, std::nullopt, (at::ScalarType)d["x_dtype"].toInt());
-        return {dx, dw, db, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+        return {dx, dw, db, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
     }
 };
 
+// part_n: see linear_fwd_impl; -1 takes the training forward whatever is recorded.
 at::Tensor linear(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
-                  int64_t bs, bool quantize_input, bool quantize_grad) {
+                  int64_t bs, bool quantize_input, bool quantize_grad, int64_t part_n) {
     // the autograd node records every tensor argument's device, so a missing
     // bias travels as an empty tensor (no storage) that forward() treats as absent
     const bool has_bias = bias && bias->defined();
     // what Function::apply tests before it makes the node a backward can reach
-    const bool train = at::GradMode::is_enabled() &&
-                       (input.requires_grad() || weight.requires_grad() || (has_bias && bias->requires_grad()));
+    const bool train = part_n < 0 || (at::GradMode::is_enabled() &&
+                                  (input.requires_grad() || weight.requires_grad() ||
+                                   (has_bias && bias->requires_grad())));
     return LinearFunction::apply(input, weight, has_bias ? *bias : at::empty({0}, input.options()), bs,
-                                 quantize_input, quantize_grad, has_bias, train);
+                                 quantize_input, quantize_grad, has_bias, train, part_n);
 }
 
 // axs6_nf5_fused_linear (axs/unified/triton_kernels.py:385-482) for input (*, K)
@@ -579,7 +585,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("weight"), py::arg("bias"), py::arg("ndim"), py::arg("eps"));
     m.def("linear", &linear, "FQ(input) FQ(weight)^T + bias with the quantized backward (autograd node)",
           py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("block_size"), py::arg("quantize_input"),
-          py::arg("quantize_grad"));
+          py::arg("quantize_grad"), py::arg("part_n") = 0);
     m.def("fused_linear", &fused_linear, "the fused linear of small outputs (block size 32, no autograd)",
           py::arg("input"), py::arg("weight"), py::arg("bias"), py::arg("quantize_input"));
     m.def("linear_infer", &linear_infer, "the forward alone: FQ(input) FQ(weight)^T + bias (no autograd)",

@@ -286,6 +286,18 @@ int axs6_nf5_linear_infer(const void* x, const void* w, const void* bias, int32_
                           int32_t dtype, int64_t M, int64_t N, int64_t K, int32_t block_size,
                           int32_t quantize_input, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same for a w of several weights of part_n rows each, stacked: every output
+ * has the bits that axs6_nf5_linear_infer gives for its own weight (the order of
+ * a sum follows the weight's size).  The query is -1 too where the weights do
+ * better one by one (one or two rows).
+ * Replaces: the q/k/v projections of modules_unified.py:235-243 as one. */
+int64_t axs6_nf5_linear_infer_stacked_workspace(int64_t M, int64_t N, int64_t K, int64_t part_n, int32_t dtype,
+                                                int32_t block_size);
+int axs6_nf5_linear_infer_stacked(const void* x, const void* w, const void* bias, int32_t bias_dtype, void* y,
+                                  int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t part_n,
+                                  int32_t block_size, int32_t quantize_input, void* workspace,
+                                  int64_t workspace_bytes, void* stream);
+
 /* Device workspace (bytes) axs6_nf5_linear_backward needs for the requested
  * gradients. */
 size_t axs6_nf5_linear_backward_workspace(int64_t M, int64_t N, int64_t K, int32_t need_dx,

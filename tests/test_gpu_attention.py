@@ -239,3 +239,35 @@ def test_self_attention_groups_projections():
     h.remove()
     assert calls == [1] and orig is u.functional_unified.axs_linear_unified
     assert torch.equal(y_grouped, y_sep)
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("m,K,sizes,dt", [
+    (64, 1280, (1280, 1280, 1280), torch.float32),    # packed one by one, large enough for the other form stacked
+    (64, 2048, (2048, 2048, 2048), torch.float32),    # stacked in the other form, with the splits of one
+    (128, 2080, (2050, 2050), torch.bfloat16),        # the same, tiles across the weights' border
+    (33, 4096, (4096, 4096, 4096), torch.float32),    # one by one
+    (100, 1024, (4096, 1024, 1024), torch.bfloat16),  # one of them
+    (1, 4096, (1024, 1024, 1024), torch.float32),     # one row: the waves per weight row follow the size
+    (2, 768, (768, 768, 768), torch.float16),
+    (200, 1000, (1024, 512, 512), torch.float32),     # none: stacked
+], ids=str)
+def test_linear_group_matches_separate_without_gradients(m, K, sizes, dt, bias):
+    from axs.unified import axs_linear_group_unified, axs_linear_unified
+
+    g = torch.Generator().manual_seed(m + K)
+    x = torch.randn(m, K, generator=g).to(DEV, dt)
+    ws = [(torch.randn(n, K, generator=g) * K ** -0.5).to(DEV, dt) for n in sizes]
+    bs = [torch.randn(n, generator=g).to(DEV, dt) for n in sizes] if bias else None
+    with torch.no_grad():
+        ys = axs_linear_group_unified(x, ws, bs)
+        sep = [axs_linear_unified(x, w, bs[i] if bias else None) for i, w in enumerate(ws)]
+    assert [tuple(y.shape) for y in ys] == [(m, n) for n in sizes]
+    assert all(torch.equal(y, s) for y, s in zip(ys, sep))
+    # one of them recorded
+    ws[1].requires_grad_(True)
+    ys = axs_linear_group_unified(x, ws, bs)
+    sep = [axs_linear_unified(x, w, bs[i] if bias else None) for i, w in enumerate(ws)]
+    assert all(torch.equal(y, s) for y, s in zip(ys, sep))
+    ys[1].sum().backward()
+    assert ws[1].grad is not None
