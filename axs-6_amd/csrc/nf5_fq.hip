@@ -247,6 +247,9 @@ template <int DT> using UnalignedVec = typename std::conditional<DT == AXS6_F32,
 // ones 31.9 and 45.4 us in the first line), plain loads (streaming ones 29.0
 // and 41.1: neighbouring waves share a line).
 constexpr int kRowsUnroll = 3;
+// Workgroups along x: a grid dimension holds under 2^32 threads, which rows of 65
+// values reach at 139 GB; more go along y.
+constexpr int64_t kRowsGridX = (int64_t)1 << 22;
 
 template <int DT, int BS, bool STOCH>
 __global__ __launch_bounds__(kThreads) void fq_rows_kernel(const typename Elem<DT>::S* __restrict__ x,
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(kThreads) void fq_rows_kernel(const typename Elem<D
     __shared__ uint32_t band_w[kBandSize / 4];
     const uint8_t* band_s = reinterpret_cast<const uint8_t*>(band_w);
     const int tid = threadIdx.x;
-    const int64_t l0 = (int64_t)blockIdx.x * (kThreads * kRowsUnroll);
+    const int64_t l0 = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (kThreads * kRowsUnroll);
     int64_t row[kRowsUnroll], col[kRowsUnroll];
     u32x4 raw[kRowsUnroll];
     {
@@ -963,7 +966,9 @@ void launch_fq_typed(const void* x, void* y, int64_t rows, int64_t cols, bool st
     const bool four = cols % 4 == 0 && (uintptr_t)x % (4 * esize) == 0 && (uintptr_t)y % (4 * esize) == 0;
     if (cols >= 4 * kRowsMinCols || (cols >= kRowsMinCols && !four)) {
         const int64_t gp = (cols + BS - 1) / BS * (BS / V), groups = rows * gp;
-        const dim3 grid((unsigned)((groups + kThreads * kRowsUnroll - 1) / (kThreads * kRowsUnroll)));
+        const int64_t need = (groups + kThreads * kRowsUnroll - 1) / (kThreads * kRowsUnroll);
+        const dim3 grid((unsigned)(need < kRowsGridX ? need : kRowsGridX),
+                        (unsigned)((need + kRowsGridX - 1) / kRowsGridX));
         if (stochastic)
             fq_rows_kernel<DT, BS, true><<<grid, kThreads, 0, st>>>((const S*)x, (S*)y, groups, cols, gp, t.lut, t.band, seed,
                                                                     seed_dev, offset);

@@ -47,3 +47,32 @@ def test_fq_ragged_rows(cols, dt):
         u = oracle.uniform(SEED, 0, x.numel())
         got = hip_fused_fake_quantize(xd, bs, "stochastic", seed=SEED).cpu()
         assert torch.equal(_bits(got), _bits(_want(x, bs, u))), (rows, bs)
+
+
+def test_fq_ragged_rows_past_one_grid_dimension():
+    """More groups than the threads of one grid dimension (2^32, three groups a
+    thread): 140 GB of rows of 65 values, in place; rows around the border of a
+    dimension's share, at the 2^32 threads and at the end."""
+    from axs import _lib
+
+    cols, per_row = 65, 12                       # bf16, block 32: 12 groups of 8 values
+    rows = 3 * 2 ** 32 // per_row + 1000
+    free, _ = torch.cuda.mem_get_info()
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < rows * cols * 2 + (2 << 30):
+        pytest.skip(f"needs 142 GB of device memory, {free >> 30} GiB are free")
+    x = torch.zeros(rows, cols, dtype=torch.bfloat16, device=DEV)
+    g = torch.Generator().manual_seed(3)
+    share = 3 * 256 * 2 ** 22 // per_row         # rows of one step along y
+    spots = [0, share - 4, 2 * share - 4, 3 * 2 ** 32 // per_row - 4, rows - 8]
+    want = []
+    for r in spots:
+        v = torch.randn(8, cols, generator=g).bfloat16()
+        x[r : r + 8].copy_(v)
+        want.append(_want(v, 32))
+    _lib.call("axs6_nf5_fake_quantize", x.data_ptr(), x.data_ptr(), _lib.DTYPE_CODE[x.dtype], rows, cols, 32, 0, 0, 0,
+              None, _lib.stream_of(x))
+    for r, w in zip(spots, want):
+        assert torch.equal(_bits(x[r : r + 8].cpu()), _bits(w)), r
+    del x
+    torch.cuda.empty_cache()
