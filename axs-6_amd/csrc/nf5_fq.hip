@@ -463,9 +463,9 @@ __device__ __forceinline__ int quant_values(float (&f)[V], uint32_t m, const flo
 // U vectors of a workgroup's contiguous run are loaded together (U == 1: the
 // next one is loaded while one is processed).  The loads in flight bound it:
 // f32, device us, four or more tensors in turn, one ahead -> U = 2: codes
-// alone 11008 x 4096 54.7 -> 47.9, 32768 x 4096 150.6 -> 130.8 (5.0 -> 6.2
-// TB/s); with the FQ output 78.5 -> 76.9, 2048 x 2048 10.1 -> 8.5.  Four are
-// slower (codes alone 49.4).  16-bit vectors hold twice the work per load and
+// alone 11008 x 4096 51.3 -> 47.7, 32768 x 4096 150.6 -> 130.8 (5.0 -> 6.2
+// TB/s); with the FQ output 2048 x 2048 9.9 -> 9.1, larger ones the other way
+// (kQuantOneVecs).  Four are slower (codes alone 49.4).  16-bit vectors hold twice the work per load and
 // keep U = 1 (8192 x 4096 bf16 with the FQ output 37.7, U = 2 38.9).
 template <int DT, int BS, bool STOCH, int U>
 __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(
@@ -1013,9 +1013,14 @@ void launch_fq(const void* x, void* y, int64_t rows, int64_t cols, int bs, bool 
 // f32 vectors from which quantize_vec_kernel without an FQ output makes two
 // iterations per workgroup, which halves the table staging; us, one -> two:
 // 4096 x 2048 12.4 -> 11.8, 4096 x 4096 22.8 -> 20.2, 8192 x 4096 40.6 -> 36.8;
-// 2048 x 2048 7.3 -> 8.0 (too few workgroups then).  With an FQ output one is
-// faster or equal up to 8192 x 4096 (2048 x 2048 8.5 against 10.6).
+// 2048 x 2048 7.3 -> 8.0 (too few workgroups then).
 constexpr int64_t kQuantTwiceVecs = (int64_t)2 << 20;
+// f32 vectors from which the quantize with an FQ output loads one vector ahead
+// (two iterations per workgroup) instead of two together (one iteration): its
+// stores, 10 of 14 bytes a value, bound it; us, two together -> one ahead: 3072 x
+// 2048 13.3 -> 14.6, 4096 x 2048 16.9 -> 17.8, 4096 x 4096 31.4 -> 31.4, 6144 x 4096
+// 44.9 -> 44.1, 8192 x 4096 59.0 -> 57.7, 11008 x 4096 77.4 -> 75.9.
+constexpr int64_t kQuantOneVecs = (int64_t)4 << 20;
 // Groups of four from which dequantize_vec_kernel loads two per lane; us, one ->
 // two: 11008 x 4096 54.3 -> 44.4 (5.0 -> 6.1 TB/s), 4096 x 2048 12.4 -> 11.1, 1448 x
 // 1024 3.8 -> 3.5; 1024 x 1024 3.1 -> 3.3 (four workgroups per CU become two).
@@ -1031,13 +1036,22 @@ void launch_quant_typed(const void* x, int64_t rows, int64_t cols, bool stochast
     if (cols % BS == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)codes % V == 0 && (uintptr_t)signs % V == 0 &&
         (uintptr_t)fq % 16 == 0) {
         const int64_t n_vec = rows * cols / V;
-        constexpr int U = DT == AXS6_F32 ? 2 : 1;
-        const int per = U == 1 || (!fq && n_vec >= kQuantTwiceVecs) ? 2 : 1;   // iterations per workgroup
-        const dim3 grid((unsigned)capped_grid(n_vec, (int64_t)kThreads * U * per));
-        if (stochastic)
-            quantize_vec_kernel<DT, BS, true, U><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
-        else
-            quantize_vec_kernel<DT, BS, false, U><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
+        auto run = [&](auto u) {
+            constexpr int U = decltype(u)::value;
+            const int per = U == 1 || (!fq && n_vec >= kQuantTwiceVecs) ? 2 : 1;   // iterations per workgroup
+            const dim3 grid((unsigned)capped_grid(n_vec, (int64_t)kThreads * U * per));
+            if (stochastic)
+                quantize_vec_kernel<DT, BS, true, U><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
+            else
+                quantize_vec_kernel<DT, BS, false, U><<<grid, kThreads, 0, st>>>((const S*)x, n_vec, t.lut, t.band, t.rev, seed, seed_dev, offset, exps, codes, signs, (S*)fq);
+        };
+        if constexpr (DT == AXS6_F32) {
+            if (!fq || n_vec < kQuantOneVecs) {
+                run(std::integral_constant<int, 2>());
+                return;
+            }
+        }
+        run(std::integral_constant<int, 1>());
         return;
     }
     const int64_t nblk = (cols + BS - 1) / BS;

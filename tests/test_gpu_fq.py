@@ -309,6 +309,18 @@ def test_codec_vector_runs(shape):
     assert bits_equal(fq, oracle.fake_quantize(x.numpy(), 8, u))
 
 
+@pytest.mark.parametrize("rows", [16383, 16385])
+def test_quantize_fq_output_vector_choice(rows):
+    """f32 with the FQ output on both sides of the size from which it loads one
+    vector ahead instead of two together (16384 rows of 1024)."""
+    x = config2_input((rows, 1024), 84)
+    e, c, s, fq = _quant(x.to(DEV), 32, "nearest", 0)
+    oe, oc, os_ = oracle.quantize(x.numpy(), 32)
+    assert np.array_equal(e.reshape(oe.shape), oe) and np.array_equal(c.reshape(oc.shape), oc)
+    assert np.array_equal(s.reshape(os_.shape), os_)
+    assert bits_equal(fq, oracle.fake_quantize(x.numpy(), 32))
+
+
 # Row-segment kernel (fq_rows_kernel): rows of >= 64 values that do not tile
 # into 16-byte vectors of whole blocks -- a ragged last block, or a view whose
 # start is off 16-byte alignment.  One segment per wave (64 columns), four
