@@ -109,13 +109,19 @@ __device__ __forceinline__ bool vec_own(int64_t vi, int64_t at, int e) {
 // and the backward's x and dy, read for the last time, by nontemporal loads
 // (the forward's x by plain ones: a backward reads it again).  Plain stores
 // leave the 256 MiB last-level cache dirty lines whose write-back the next
-// kernels pay.  us, forward and forward + backward, three tensors in turn,
-// plain -> streaming: 8192 x 4096 f32 53.5, 143.0 -> 50.3, 118.7; 16384 x 2048
-// f32 49.2, 137.8 -> 48.3, 117.7; 8192 x 4096 bf16 32.2, 95.5 -> 22.5, 85.8;
-// 8192 x 1024 f32 12.5, 39.2 -> 12.1, 33.4.  Below, a tensor stays in the cache
-// for what reads it next, and streaming loads lose (8192 x 1024 bf16, 16 MiB:
-// 27.9 -> 29.9).
-constexpr int64_t kLnStreamBytes = (int64_t)32 << 20;
+// kernels pay; below this size what reads y or dx next finds it in the cache.
+// us, three inputs in turn, plain -> streaming:
+//                       forward +      forward and    forward, linear N = cols,
+//                       backward       fake-quantize  backward, dx added to
+//   8192 x 1024 f32     36.0 -> 33.2    25.3 -> 26.1    190.9 -> 192.1
+//   8192 x 2048 f32     74.3 -> 68.1    45.0 -> 46.2    417.6 -> 425.1
+//   8192 x 3072 f32    103.3 -> 95.9    70.6 -> 74.8    732.1 -> 738.3
+//   8192 x 4096 f32    142.7 -> 118.2   92.2 -> 97.3   1012.7 -> 997.2
+//   16384 x 3072 bf16  139.0 -> 137.7   83.1 -> 88.1   1180.8 -> 1190.0
+//   16384 x 4096 bf16  165.3 -> 155.9   98.2 -> 105.3  1691.3 -> 1687.0
+//   16384 x 4096 f32   278.6 -> 238.4  180.0 -> 186.4
+// (the norm alone reads nothing of what it wrote: the last column decides).
+constexpr int64_t kLnStreamBytes = (int64_t)128 << 20;
 
 struct LnArgs {
     const void* x; const void* dy; const void* gamma; const void* beta;

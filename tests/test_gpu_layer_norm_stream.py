@@ -1,10 +1,10 @@
-"""The LayerNorm vector kernels' streaming instances (tensors of 32 MiB and
+"""The LayerNorm vector kernels' streaming instances (tensors of 128 MiB and
 more: nontemporal stores and last-use loads) and the backward's next-row
-prefetch, at the edges: just below and at 32 MiB, row counts that leave a
+prefetch, at the edges: just below and at 128 MiB, row counts that leave a
 partial chunk or fewer rows than workgroups, and rows whose last vector group
-is partial; and the ragged instances (rows of no whole number of vectors).  Against float64 F.layer_norm; the bars are those of the kernels'
-other test (f32: rounding of sums of up to 16K terms; 16-bit: one rounding of
-the result)."""
+is partial; and the ragged instances (rows of no whole number of vectors).
+Against float64 F.layer_norm; the bars are those of the kernels' other test
+(f32: rounding of sums of up to 16K terms; 16-bit: one rounding of the result)."""
 from __future__ import annotations
 
 import pytest
@@ -19,12 +19,24 @@ TOL = {torch.float32: 2e-6, torch.bfloat16: 8e-3, torch.float16: 1e-3}
 
 # (rows, cols, dtype)
 CASES = [
-    (8192, 1024, torch.float32),     # 32 MiB, a wave per row
-    (8191, 1024, torch.float32),     # one row less: not streamed
+    (32768, 1024, torch.float32),    # 128 MiB, a wave per row
+    (32767, 1024, torch.float32),    # one row less: not streamed
+    (131075, 260, torch.float32),    # streamed, last group of one vector
+    (8209, 4100, torch.float32),     # streamed, a workgroup per row
+    (4099, 8188, torch.float32),     # streamed, prefetch in f32, last group short
+    (16387, 4104, torch.bfloat16),   # streamed, prefetch
+    (8193, 8192, torch.float16),
+    (65539, 1032, torch.bfloat16),
+    (262145, 264, torch.float16),
+    (16400, 4097, torch.bfloat16),   # streamed, ragged
+    (65600, 515, torch.float32),     # streamed, ragged, a wave per row
+    # the same forms below that size
+    (8192, 1024, torch.float32),
+    (8191, 1024, torch.float32),
     (32771, 260, torch.float32),     # a wave per row, last group of one vector
     (2053, 4100, torch.float32),     # a workgroup per row, last group of one vector
     (1025, 8188, torch.float32),     # prefetch in f32, last group short
-    (4099, 4104, torch.bfloat16),    # prefetch, streamed, last group of one vector
+    (4099, 4104, torch.bfloat16),    # prefetch, last group of one vector
     (2049, 8192, torch.float16),
     (16387, 1032, torch.bfloat16),
     (65537, 264, torch.float16),     # a wave per row, 16-bit
@@ -40,8 +52,8 @@ CASES = [
     (9, 8191, torch.float32),        # the longest ragged vector row
     (31, 2047, torch.float16),
     (9, 8191, torch.bfloat16),
-    (4100, 4097, torch.bfloat16),    # streamed
-    (16400, 515, torch.float32),     # streamed, a wave per row
+    (4100, 4097, torch.bfloat16),
+    (16400, 515, torch.float32),     # a wave per row
 ]
 
 
