@@ -268,7 +268,8 @@ __device__ __forceinline__ f32x4m mfma_elem(u32x4 a, u32x4 b, f32x4m c) {
 }
 
 constexpr int kXSlabs = 3;
-template <int DT, int BM> constexpr int infer_waves() { return BM >= 128 || (DT == AXS6_F32 && BM == 64) ? 2 : 4; }
+// Waves per SIMD that an instance's registers are kept to; a workgroup is two.
+constexpr int infer_waves(int dtype, int bm) { return bm >= 128 || (dtype == AXS6_F32 && bm == 64) ? 2 : 4; }
 
 constexpr size_t infer_lds(int BM) {
     return (size_t)kXSlabs * BM * kIK * 2 + 2 * kIN * kIK * 2 + 2 * 2 * kIN * sizeof(float);
@@ -425,7 +426,7 @@ __global__ __launch_bounds__(256) void infer_reduce_kernel(InferK k) {
 
 // MW x NW waves over the BM x 128 tile.
 template <int DT, int BM, int MW, int NW>
-__global__ __launch_bounds__(kIThreads, (infer_waves<DT, BM>())) void infer_gemm_kernel(InferK k) {
+__global__ __launch_bounds__(kIThreads, infer_waves(DT, BM)) void infer_gemm_kernel(InferK k) {
 #if defined(__HIP_DEVICE_COMPILE__)
     static_assert(MW * NW == 8, "eight waves");
     constexpr int TM = BM / (16 * MW), TN = kIN / (16 * NW);
@@ -671,13 +672,13 @@ struct InferPlan { int bm, steps, splits; size_t xq, sx, again, refs, partial, t
 // us, packed path / this one:
 //            M x K x N          bf16          f32
 //     16 x 4096 x 11008   67.8 / 35.9    71.3 / 48.9
-//     64 x 4096 x 4096    42.4 / 23.5    46.8 / 30.7
-//    128 x 4096 x 4096    43.5 / 27.8    47.6 / 35.8
+//     64 x 4096 x 4096    42.4 / 22.5    46.8 / 29.8
+//    128 x 4096 x 4096    43.5 / 27.8    47.6 / 33.5
 //    256 x 4096 x 4096    43.0 / 34.8    48.0 / 50.8
-//    256 x 4096 x 11008   75.5 / 66.5    84.0 / 124.7
+//    256 x 4096 x 11008   75.5 / 61.3    84.0 / 124.7
 //    256 x 11008 x 4096  104.8 / 55.3   111.7 / 103.7
 //    512 x 4096 x 4096    44.8 / 47.4    49.4 / 82.2
-//     64 x 2048 x 2048         -         26.6 / 24.8
+//     64 x 2048 x 2048         -         26.6 / 22.3
 //    128 x 2048 x 2048         -         26.2 / 27.8
 //    128 x 1024 x 1024    17.3 / 17.4    17.7 / 19.5
 //     16 x 512 x 11008         -         16.6 / 19.2
@@ -693,8 +694,11 @@ bool infer_plan(int64_t M, int64_t N, int64_t K, int64_t part_n, int dtype, Infe
     const int64_t tiles = (N + kIN - 1) / kIN, part_tiles = (part_n + kIN - 1) / kIN;
     const int64_t steps = (K + kIK - 1) / kIK;
     // K splits: rounds of workgroups times the steps of each, the fill of its
-    // pipeline (about 4 steps) and the partial sums' traffic (about 1 step per split)
-    const int64_t slots = p->bm >= 128 ? 256 : 512;
+    // pipeline (about 4 steps) and the partial sums' traffic (about 1 step per split).
+    // The slots are the workgroups that fit the CUs: counted as 512 where one
+    // fits a CU (f32 of 64 rows), twice the splits ran in two rounds: 64 x 11008 x
+    // 4096 71 us against 53, 48 x 4096 x 6144 44 against 34.5.
+    const int64_t slots = 256 * infer_waves(dtype, p->bm) / 2;
     int64_t s = 1, best = INT64_MAX;
     for (int64_t c = 1; c <= 16 && c <= steps / 4 + 1; ++c) {
         const int64_t cost = ((part_tiles * c + slots - 1) / slots) * (((steps + c - 1) / c) + 4) + (c > 1 ? 2 + c : 0);

@@ -214,3 +214,15 @@ def test_fused_linear_split_workspace_and_arguments_without_device():
     assert rc == 1 and "block_size" in msg
     rc, _ = _status(name, fake, fake, None, fake, None, _lib.F32, 0, 64, 2048, 32, 1, None)
     assert rc == 0      # nothing to compute
+
+
+def test_linear_infer_split_fits_the_card_without_device():
+    """The K split of an instance of which one workgroup fits a CU (f32 from 33
+    rows, 16-bit from 65) counts on 256 of them: more, and a second round runs.
+    Seen from the workspace, whose partial tiles are rows x 128 floats each."""
+    q = _lib.lib().axs6_nf5_linear_infer_workspace
+    for dtype, m, tile in ((_lib.F32, 64, 64), (_lib.F32, 33, 64), (_lib.F32, 100, 128), (_lib.BF16, 100, 128)):
+        for N, K in ((8192, 4096), (4096, 4096), (4096, 11008), (6144, 4096)):
+            partial = q(m, N, K, dtype, 32) - m * K * 2
+            # the row exponents of f32 partial tiles: 513 bytes a tile
+            assert 0 < partial <= 256 * (tile * 128 * 4 + 128 * 4 + 4) + 2048, (dtype, m, N, K, partial)
