@@ -216,6 +216,26 @@ def test_fused_linear_split_workspace_and_arguments_without_device():
     assert rc == 0      # nothing to compute
 
 
+def test_linear_infer_rule_without_device():
+    """The host-only query of the forward without gradients, (M, N, K, dtype,
+    block_size): bytes of workspace, or -1 where there is no such form."""
+    q = _lib.lib().axs6_nf5_linear_infer_workspace
+    F, B, H = _lib.F32, _lib.BF16, _lib.F16
+    # one and two rows: while FQ(X) in f32 fits 48 KiB, any N
+    assert q(1, 1, 32, F, 32) == 0 and q(1, 4096, 12288, B, 32) == 0 and q(2, 4096, 6144, H, 32) == 0
+    assert q(1, 4096, 12320, F, 32) == -1 and q(2, 4096, 6176, F, 32) == -1
+    # 3 rows up: K >= 1024, 4M weight values, and rows by type and weight
+    assert q(3, 4096, 1024, F, 32) > 0 and q(3, 4095, 1024, F, 32) == -1 and q(3, 8192, 992, F, 32) == -1
+    assert q(64, 4096, 1024, F, 32) > 0 and q(65, 4096, 1024, F, 32) == -1
+    assert q(128, 4096, 1024, B, 32) > 0 and q(129, 4096, 1024, B, 32) == -1
+    assert q(128, 4096, 2048, F, 32) > 0 and q(129, 4096, 2048, F, 32) == -1
+    assert q(256, 4096, 2048, H, 32) > 0 and q(257, 4096, 2048, H, 32) == -1
+    # other blocks, ragged K, empty or negative sizes, unknown types, operands past 2 GiB
+    assert q(64, 4096, 4096, F, 16) == -1 and q(64, 4096, 4100, F, 32) == -1 and q(64, 4096, 4096, 7, 32) == -1
+    assert q(0, 4096, 4096, F, 32) == -1 and q(64, 0, 4096, F, 32) == -1 and q(-1, 4096, 4096, F, 32) == -1
+    assert q(64, 1 << 20, 1024, F, 32) == -1 and q(64, 1 << 20, 512, B, 32) == -1
+
+
 def test_linear_infer_split_fits_the_card_without_device():
     """The K split of an instance of which one workgroup fits a CU (f32 from 33
     rows, 16-bit from 65) counts on 256 of them: more, and a second round runs.
@@ -226,3 +246,53 @@ def test_linear_infer_split_fits_the_card_without_device():
             partial = q(m, N, K, dtype, 32) - m * K * 2
             # the row exponents of f32 partial tiles: 513 bytes a tile
             assert 0 < partial <= 256 * (tile * 128 * 4 + 128 * 4 + 4) + 2048, (dtype, m, N, K, partial)
+
+
+def test_linear_infer_stacked_rule_without_device():
+    """(M, N, K, part_n, ...): the weight's own rule and split, for N rows."""
+    q = _lib.lib().axs6_nf5_linear_infer_stacked_workspace
+    one = _lib.lib().axs6_nf5_linear_infer_workspace
+    F, B = _lib.F32, _lib.BF16
+    assert q(64, 2048, 2048, 2048, F, 32) == one(64, 2048, 2048, F, 32) > 0
+    # three times the partial tiles of one, X once
+    x = 64 * 2048 * 2
+    assert abs((q(64, 6144, 2048, 2048, B, 32) - x) - 3 * (one(64, 2048, 2048, B, 32) - x)) <= 3 * 512
+    # one weight is under the rule's size, two of them are not
+    assert q(64, 2560, 1280, 1280, F, 32) == -1 and one(64, 2560, 1280, F, 32) == -1
+    assert q(64, 3840, 1280, 1280, F, 32) == -1 and one(64, 3840, 1280, F, 32) > 0
+    # one and two rows: the waves of a row follow the weight's size
+    assert q(1, 4096, 4096, 4096, F, 32) == 0 and q(1, 12288, 4096, 4096, F, 32) == -1
+    assert q(64, 2048, 2048, 0, F, 32) == -1 and q(64, 2048, 2048, 4096, F, 32) == -1
+
+
+def test_linear_infer_arguments_without_device():
+    fake = 4096       # never dereferenced: the checks fail first
+    F = _lib.F32
+
+    def call(x=fake, w=fake, bias=None, bias_dtype=F, y=fake, dtype=F, M=64, N=4096, K=4096, bs=32, ws=fake, n=1 << 40):
+        return _status("axs6_nf5_linear_infer", x, w, bias, bias_dtype, y, dtype, M, N, K, bs, 1, ws, n, None)
+
+    assert call(dtype=9)[0] == 1 and "dtype" in call(dtype=9)[1]
+    rc, msg = call(bias=fake, bias_dtype=5)
+    assert rc == 1 and "dtype code 5" in msg
+    rc, msg = call(bs=16)
+    assert rc == 1 and "block_size" in msg
+    assert call(M=-1)[0] == 1 and call(K=-32)[0] == 1
+    assert call(M=0, x=None, y=None)[0] == 0 and call(N=0, w=None)[0] == 0      # nothing to compute
+    for a in (dict(M=512), dict(K=4100), dict(N=64), dict(M=2, K=8192)):         # no such form
+        rc, msg = call(**a)
+        assert rc == 2 and "no inference form" in msg, a
+    for a in (dict(x=None), dict(w=None), dict(y=None)):
+        rc, msg = call(**a)
+        assert rc == 1 and "null" in msg, a
+    for a in (dict(x=fake + 4), dict(w=fake + 8)):
+        rc, msg = call(**a)
+        assert rc == 1 and "16-byte aligned" in msg, a
+    need = _lib.lib().axs6_nf5_linear_infer_workspace(64, 4096, 4096, F, 32)
+    for a in (dict(ws=None), dict(ws=fake + 4), dict(n=need - 1)):
+        rc, msg = call(**a)
+        assert rc == 1 and "workspace" in msg, a
+    # the stacked entry's part
+    rc, msg = _status("axs6_nf5_linear_infer_stacked", fake, fake, None, F, fake, F, 64, 4096, 4096, 8192, 32, 1, fake,
+                      1 << 40, None)
+    assert rc == 2 and "no inference form" in msg

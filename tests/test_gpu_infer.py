@@ -236,3 +236,28 @@ def test_infer_subnormal_values_round_once(m, dt):
     k = torch.arange(N) % K
     want = (vq[:, k].float() * dq[torch.arange(N), k].float()).to(dt)
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("m", [1, 40])
+@pytest.mark.parametrize("dt,bt", [(torch.bfloat16, torch.float32), (torch.float16, torch.float64),
+                                   (torch.float32, torch.bfloat16), (torch.float32, torch.float64)], ids=str)
+def test_infer_bias_of_another_type(m, dt, bt):
+    """A bias of another floating type is added in its own value (float64: as
+    float32), and broadcasts as F.linear's."""
+    x, w, _ = _inputs(m, 1024, 4100, dt, 31)
+    assert _form(m, 1024, 4100, dt)
+    b = (torch.randn(4100, generator=torch.Generator().manual_seed(32)) * 3.0).to(bt)
+    want = _exact(x, w, b)
+    y = _infer(x, w, b)
+    assert y.dtype == dt
+    assert oracle.rel_l2(y.float().cpu().numpy(), want) <= BAR[dt]
+    y = _infer(x, w, b[:1])
+    assert oracle.rel_l2(y.float().cpu().numpy(), _exact(x, w, b[:1])) <= BAR[dt]
+    with pytest.raises(RuntimeError, match="broadcast"):
+        _infer(x, w, b[:7])
+
+
+def test_infer_float64_is_computed_in_float32():
+    x, w, b = _inputs(40, 1024, 4100, torch.float32, 33)
+    y = _infer(x.double(), w.double(), b.double())
+    assert y.dtype == torch.float64 and torch.equal(y, _infer(x, w, b).double())
