@@ -682,12 +682,17 @@ struct InferPlan { int bm, steps, splits; size_t xq, sx, again, refs, partial, t
 //    128 x 2048 x 2048         -         26.2 / 27.8
 //    128 x 1024 x 1024    17.3 / 17.4    17.7 / 19.5
 //     16 x 512 x 11008         -         16.6 / 19.2
+// One and two rows come here where FQ(X) is past the streamed form's LDS (one
+// row of 12288 values, two of 6144): 2 x 11008 x 4096 bf16 100.8 / 39.9, 1 x 14336 x
+// 4096 f32 140.2 / 67.4.
+// A K off 32 and blocks of 8 and 16 stay with the packed path: 64 x 4096 x 4096
+// f32 29.7 here, 46.6 there in blocks of 16 and 55.7 at K 4100.
 // part_n: the rows of one of the weights that make up W, whose plan it takes (N:
 // W is one weight).
 bool infer_plan(int64_t M, int64_t N, int64_t K, int64_t part_n, int dtype, InferPlan* p) {
     const bool f32 = dtype == AXS6_F32;
     const int64_t most = part_n * K >= (int64_t)1 << 23 ? (f32 ? 128 : 256) : (f32 ? 64 : 128);
-    if (M < 3 || M > most || K < 1024 || part_n * K < (int64_t)1 << 22) return false;
+    if (M < 1 || M > most || K < 1024 || part_n * K < (int64_t)1 << 22) return false;
     // 32-bit buffer offsets
     if (N * K * (f32 ? 4 : 2) >= (int64_t)kOob || M * (K + kGemmK) * 2 >= (int64_t)kOob) return false;
     p->bm = M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256;

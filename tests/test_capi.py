@@ -221,9 +221,10 @@ def test_linear_infer_rule_without_device():
     block_size): bytes of workspace, or -1 where there is no such form."""
     q = _lib.lib().axs6_nf5_linear_infer_workspace
     F, B, H = _lib.F32, _lib.BF16, _lib.F16
-    # one and two rows: while FQ(X) in f32 fits 48 KiB, any N
+    # one and two rows: while FQ(X) in f32 fits 48 KiB, any N and no workspace
     assert q(1, 1, 32, F, 32) == 0 and q(1, 4096, 12288, B, 32) == 0 and q(2, 4096, 6144, H, 32) == 0
-    assert q(1, 4096, 12320, F, 32) == -1 and q(2, 4096, 6176, F, 32) == -1
+    assert q(1, 4096, 12320, F, 32) > 0 and q(2, 4096, 6176, F, 32) > 0          # past it the other form
+    assert q(1, 340, 12320, F, 32) == -1 and q(2, 4096, 992, F, 32) == 0
     # 3 rows up: K >= 1024, 4M weight values, and rows by type and weight
     assert q(3, 4096, 1024, F, 32) > 0 and q(3, 4095, 1024, F, 32) == -1 and q(3, 8192, 992, F, 32) == -1
     assert q(64, 4096, 1024, F, 32) > 0 and q(65, 4096, 1024, F, 32) == -1
@@ -279,7 +280,7 @@ def test_linear_infer_arguments_without_device():
     assert rc == 1 and "block_size" in msg
     assert call(M=-1)[0] == 1 and call(K=-32)[0] == 1
     assert call(M=0, x=None, y=None)[0] == 0 and call(N=0, w=None)[0] == 0      # nothing to compute
-    for a in (dict(M=512), dict(K=4100), dict(N=64), dict(M=2, K=8192)):         # no such form
+    for a in (dict(M=512), dict(K=4100), dict(N=64), dict(M=2, N=340, K=12288)):         # no such form
         rc, msg = call(**a)
         assert rc == 2 and "no inference form" in msg, a
     for a in (dict(x=None), dict(w=None), dict(y=None)):

@@ -250,6 +250,7 @@ def test_self_attention_groups_projections():
     (100, 1024, (4096, 1024, 1024), torch.bfloat16),  # one of them
     (1, 4096, (1024, 1024, 1024), torch.float32),     # one row: the waves per weight row follow the size
     (2, 768, (768, 768, 768), torch.float16),
+    (2, 6400, (700, 700, 700), torch.bfloat16),       # two rows past the streamed form
     (200, 1000, (1024, 512, 512), torch.float32),     # none: stacked
 ], ids=str)
 def test_linear_group_matches_separate_without_gradients(m, K, sizes, dt, bias):

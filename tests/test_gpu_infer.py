@@ -72,7 +72,7 @@ def test_infer_streamed_rows(m, K, N, dt):
 @pytest.mark.parametrize("dt", list(BAR), ids=str)
 @pytest.mark.parametrize("m,K,N", [(3, 1056, 4030), (32, 4096, 1024), (33, 2080, 2051), (64, 1024, 4224),
                                    (65, 4128, 2049), (128, 8192, 1027), (129, 2048, 4096), (256, 3104, 2710),
-                                   (5, 1024, 65540)])
+                                   (5, 1024, 65540), (1, 14336, 2050), (2, 11008, 1027), (2, 6176, 4096)])
 def test_infer_gemm(m, K, N, dt):
     print(f"[infer gemm {dt} m={m} K={K} N={N}]", flush=True)
     x, w, b = _inputs(m, K, N, dt, K + N + m)
