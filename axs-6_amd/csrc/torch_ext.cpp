@@ -248,11 +248,12 @@ struct Fwd {
     at::ScalarType dtype;
 };
 
-// train = false: no backward will follow, so where the library has an inference
-// form for the shape it runs instead and the packed operands stay undefined;
-// part_n: the rows of one of the weights stacked in `weight` (0: it is one).
+// part_n < 0: the training forward.  Else no backward will follow, so where the
+// library has an inference form for the shape it runs instead and the packed
+// operands stay undefined; part_n is then the rows of one of the weights stacked
+// in `weight` (0: it is one).
 Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
-                    int64_t bs, bool quantize_input, bool train = true, int64_t part_n = 0) {
+                    int64_t bs, bool quantize_input, int64_t part_n = -1) {
     const char* fn = "axs_linear";
     require_device(input, fn);
     require_device(weight, fn);
@@ -268,9 +269,9 @@ Fwd linear_fwd_impl(const at::Tensor& input, const at::Tensor& weight, const std
     const int64_t vm = vec_multiple(dtype);
     at::Tensor x2 = dense(pad_last(rows2d(input, K).to(dtype), vm));
     Fwd r;
-    if (!train) {
+    if (part_n >= 0) {
         const int64_t M = x2.size(0);
-        if (part_n <= 0) part_n = N;
+        if (part_n == 0) part_n = N;
         const int64_t ws =
             axs6_nf5_linear_infer_stacked_workspace(M, N, K, part_n, dtype_code(dtype), (int32_t)bs);
         if (ws >= 0) {
@@ -380,10 +381,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> linear_bwd_impl(
 struct LinearFunction : public torch::autograd::Function<LinearFunction> {
     static at::Tensor forward(AutogradContext* ctx, const at::Tensor& input, const at::Tensor& weight,
                               const at::Tensor& bias, int64_t bs, bool quantize_input, bool quantize_grad,
-                              bool has_bias, bool train, int64_t part_n) {
+                              bool has_bias, int64_t part_n) {
         Fwd r = linear_fwd_impl(input, weight, has_bias ? std::optional<at::Tensor>(bias) : std::nullopt, bs,
-                                quantize_input, train, part_n);
-        if (!train) return r.out;   // nothing records a gradient: nothing to save
+                                quantize_input, part_n);
+        if (part_n >= 0) return r.out;   // nothing records a gradient: nothing to save
         ctx->save_for_backward({r.xq, r.sx, r.wq, r.sw});
         auto& d = ctx->saved_data;
         d["M"] = r.M; d["N"] = r.N; d["K"] = r.K; d["n_true"] = r.n_true; d["k_true"] = r.k_true;
@@ -400,7 +401,7 @@ struct LinearFunction : public torch::autograd::Function<LinearFunction> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const at::Tensor& g = grads[0];
         if (!g.defined())
-            return variable_list(9);
+            return variable_list(8);
         const auto saved = ctx->get_saved_variables();
         auto& d = ctx->saved_data;
         const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
@@ -411,22 +412,22 @@ struct LinearFunction : public torch::autograd::Function<LinearFunction> {
             d["n_true"].toInt(), d["k_true"].toInt(), (at::ScalarType)d["dtype"].toInt(), x_shape,
             (at::ScalarType)d["w_dtype"].toInt(), d["bs"].toInt(), d["quantize_grad"].toBool(), need_x, need_w,
             need_b, std::nullopt, (at::ScalarType)d["x_dtype"].toInt());
-        return {dx, dw, db, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+        return {dx, dw, db, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
     }
 };
 
-// part_n: see linear_fwd_impl; -1 takes the training forward whatever is recorded.
+// part_n: see linear_fwd_impl; a recorded gradient takes the training forward.
 at::Tensor linear(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
                   int64_t bs, bool quantize_input, bool quantize_grad, int64_t part_n) {
     // the autograd node records every tensor argument's device, so a missing
     // bias travels as an empty tensor (no storage) that forward() treats as absent
     const bool has_bias = bias && bias->defined();
     // what Function::apply tests before it makes the node a backward can reach
-    const bool train = part_n < 0 || (at::GradMode::is_enabled() &&
-                                  (input.requires_grad() || weight.requires_grad() ||
-                                   (has_bias && bias->requires_grad())));
+    if (at::GradMode::is_enabled() &&
+        (input.requires_grad() || weight.requires_grad() || (has_bias && bias->requires_grad())))
+        part_n = -1;
     return LinearFunction::apply(input, weight, has_bias ? *bias : at::empty({0}, input.options()), bs,
-                                 quantize_input, quantize_grad, has_bias, train, part_n);
+                                 quantize_input, quantize_grad, has_bias, part_n);
 }
 
 // axs6_nf5_fused_linear (axs/unified/triton_kernels.py:385-482) for input (*, K)
@@ -479,7 +480,7 @@ at::Tensor fused_linear(const at::Tensor& input, const at::Tensor& weight, const
 // The forward alone, no gradient recorded.
 at::Tensor linear_infer(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
                         int64_t bs, bool quantize_input) {
-    return linear_fwd_impl(input, weight, bias, bs, quantize_input, false).out;
+    return linear_fwd_impl(input, weight, bias, bs, quantize_input, 0).out;
 }
 
 py::tuple linear_fwd(const at::Tensor& input, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
