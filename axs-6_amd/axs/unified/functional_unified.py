@@ -90,7 +90,11 @@ def axs_linear_unified(
     """AXS-6 quantized linear: ``input (*, in) -> (*, out)``.  Runs as one C++
     autograd node (the same forward and backward as
     ``_AXSLinearUnifiedFunction``, whose Python class is kept for callers
-    that use it directly)."""
+    that use it directly).  Where no gradient is recorded, small inputs (up to
+    256 rows, by weight size) take forms that leave the weight unpacked: their
+    results agree with a recorded forward's to the operands' rounding (3e-4 at
+    one or two float32 rows, which keep float32 operands) or the order of
+    float32 sums (the others), not bit for bit."""
     return hip_linear.linear_autograd(input, weight, bias, block_size, quantize_input, quantize_grad)
 
 

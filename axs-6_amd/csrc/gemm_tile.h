@@ -1,6 +1,6 @@
 // Device building blocks of the fp16 MFMA GEMM tiles (gfx950), shared by the
-// plain GEMM (gemm_f16.hip) and the forward with streamed operand packing
-// (nf5_linear_stream.hip): the XOR-swizzled LDS slab layout, the per-wave
+// plain GEMM (gemm_f16.hip) and the linear without gradients
+// (nf5_linear_infer.hip): the XOR-swizzled LDS slab layout, the per-wave
 // accumulator tile and its 16x16x32 MFMA K-step, the epilogue that leaves
 // through LDS as whole-row-segment stores, and vmcnt waits with immediate
 // counts.

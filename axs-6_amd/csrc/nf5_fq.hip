@@ -138,7 +138,7 @@ __device__ __forceinline__ void store4(typename Elem<DT>::S* p, const float (&f)
     }
 }
 
-// Rows too short for the row-segment layout (under 64 values, or under 256
+// Rows too short for fq_rows_kernel (under 64 values, or under 256
 // with four values per lane): each wave takes R = 64 * VL / cols whole rows
 // per step, lane l holding values VL*l .. VL*l + VL-1 of the wave's
 // contiguous run of R * cols values, so loads and stores are consecutive

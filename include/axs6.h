@@ -269,9 +269,11 @@ int axs6_nf5_fused_linear_split(const void* x, const void* w, const float* bias,
                                 int32_t quantize_input, void* stream);
 
 /* Forward without gradients: y = FQ(x) FQ(w)^T + bias with the FQ values in the
- * operands' type, as axs6_nf5_linear_forward computes it (equal to its
- * operand rounding), but with no packed operands left for a backward, for the
- * shapes where that is faster.  x [M, K], w [N, K] dense and 16-byte aligned,
+ * operands' type, as axs6_nf5_linear_forward computes it, but with no packed
+ * operands left for a backward, for the shapes where that is faster.  Not bit
+ * for bit that forward: the order of the f32 sums differs, and one or two f32
+ * rows contract the f32 values themselves (that forward rounds both operands to
+ * 11 bits, 3e-4 of the result).  x [M, K], w [N, K] dense and 16-byte aligned,
  * K a multiple of 32, block_size 32; bias may be null, else N values of
  * bias_dtype.  axs6_nf5_linear_infer_workspace is a
  * host-only query: the bytes of workspace the call takes (overwritten, 16-byte

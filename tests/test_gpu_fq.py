@@ -321,10 +321,11 @@ def test_quantize_fq_output_vector_choice(rows):
     assert bits_equal(fq, oracle.fake_quantize(x.numpy(), 32))
 
 
-# Row-segment kernel (fq_rows_kernel): rows of >= 64 values that do not tile
-# into 16-byte vectors of whole blocks -- a ragged last block, or a view whose
-# start is off 16-byte alignment.  One segment per wave (64 columns), four
-# (256 columns and more), rows ending mid-segment.
+# Ragged rows (fq_rows_kernel): rows of >= 64 values that do not tile into
+# 16-byte vectors of whole blocks -- a ragged last block, or a view whose start
+# is off 16-byte alignment.  A cut last group and none, rows of fewer and more
+# groups than a workgroup steps by (256), a last workgroup partly past the
+# tensor; every length of a cut group is in test_gpu_fq_ragged.py.
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
 @pytest.mark.parametrize("bs", [8, 16, 32])
 @pytest.mark.parametrize("shape", [(300, 4100), (64, 1000), (129, 777), (5, 64), (33, 255)], ids=str)
@@ -343,7 +344,7 @@ def test_rows_kernel_bitexact(dt, bs, shape):
 @pytest.mark.parametrize("bs", [8, 32])
 def test_rows_kernel_unaligned_view(dt, bs):
     """Whole-block rows in a view one element into its buffer (the vector
-    kernel needs 16-byte alignment): the row-segment kernel, same bits."""
+    kernel needs 16-byte alignment): the ragged rows' kernel, same bits."""
     x = config2_input((256, 4096), 91 + bs).to(dt)
     buf = torch.zeros(x.numel() + 1, dtype=dt, device=DEV)
     buf[1:] = x.reshape(-1).to(DEV)
@@ -356,7 +357,7 @@ def test_rows_kernel_unaligned_view(dt, bs):
 
 def test_rows_kernel_exponent_range():
     """Blocks across the whole float32 range (subnormal, tiny, huge, inf
-    scale, NaN) through the row-segment kernel: rows of four such blocks plus
+    scale, NaN) through the ragged rows' kernel: rows of four such blocks plus
     a ragged block of seven values."""
     rng = np.random.default_rng(8)
     blocks = []
@@ -418,7 +419,7 @@ def test_short_rows_kernel_bitexact(dt, bs):
 @pytest.mark.parametrize("cols", [20, 100, 200])
 def test_short_rows_kernel_unaligned_view(dt, cols):
     """Short rows of whole 4-value groups in a view one element into its
-    buffer: one value per lane (or the row-segment kernel), same bits as the
+    buffer: one value per lane (or the ragged rows' kernel), same bits as the
     aligned tensor's four-per-lane form."""
     x = config2_input((999, cols), 5 + cols).to(dt)
     buf = torch.zeros(x.numel() + 1, dtype=dt, device=DEV)
