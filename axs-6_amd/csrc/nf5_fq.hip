@@ -221,73 +221,91 @@ __global__ __launch_bounds__(kThreads) void fq_short_kernel(const typename Elem<
 // of them still cover one contiguous KiB, over nine lines instead of eight).
 typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
 typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
-template <int DT> using UnalignedVec = typename std::conditional<DT == AXS6_F32, u32x4_at4, u32x4_at2>::type;
+typedef uint32_t u32x2_vec __attribute__((ext_vector_type(2)));
+typedef u32x2_vec u32x2_at2 __attribute__((aligned(2)));
+// what a lane of fq_rows_kernel loads: 16 bytes, or one value
+template <int DT, int VL>
+using RowsVec = std::conditional_t<VL == 1, typename Elem<DT>::S, std::conditional_t<DT == AXS6_F32, u32x4_at4, u32x4_at2>>;
 
 // Rows that do not tile into 16-byte vectors of whole blocks (a ragged last
 // block, or rows off 16-byte alignment), of kRowsMinCols or more values.  A row
-// is gp groups of V values (16 bytes), its last block's padding included, so a
-// block is BS / V neighbouring lanes of one wave whatever the row; lanes take
-// the tensor's groups in order, a thread kRowsUnroll of them, 256 apart, from
-// one division of the workgroup's first group and steps after it.  A group
-// that the row's end cuts loads the row's last V values and shifts them down
-// (zeros above: the reference's padding of the last block) and stores value
-// by value; groups past it hold zeros and store nothing.
+// is gp groups of VL values, its last block's padding included, so a block is
+// BS / VL neighbouring lanes of one wave whatever the row; lanes take the tensor's
+// groups in order, a thread U of them, 256 apart, from one division of the
+// workgroup's first group and steps after it.  A group that the row's end cuts
+// loads the row's last VL values and shifts them down (zeros above: the reference's
+// padding of the last block) and stores what the row has of it; groups past it hold
+// zeros and store nothing.
 //
-// What bounds it: VALU work per group, as in the vector kernel, and its bytes.
-// The kernel before it took one value per lane wherever a row's length or
-// start was no multiple of 4 values, and so the block's maximum, scale and
-// addresses once per value; four per lane elsewhere.  us, three inputs and
-// outputs in turn, before -> now (nearest; stochastic):
+// What bounds it: VALU work per group, as in the vector kernel, and its bytes;
+// in a tensor that leaves CUs idle, a wave's own chain from its loads to its stores.
+// So VL is 16 bytes and U is 3 (2, 4, 5 and 6: up to 8% longer) in large tensors, U is 1
+// from kRowsManyGroups down, and one value per lane under kRowsOneValue.
+// The kernel before it took one value per lane, persistent waves with the next
+// ones in flight, wherever a row's length or start was no multiple of 4 values, and
+// four elsewhere.  us, three inputs and outputs in turn, before -> now (nearest;
+// stochastic):
 //   8192 x 4095 bf16   57.0 -> 25.5   70.9 -> 39.8
 //   8192 x 4095 f32    57.9 -> 49.3   62.2 -> 50.6
 //   32768 x 1000 bf16  31.3 -> 25.9   38.5 -> 35.9
 //   2000 x 11007 bf16  35.3 -> 16.6   42.8 -> 23.5
 //   65536 x 300 f32    36.2 -> 27.2   39.2 -> 30.4
-// Three groups a thread (2, 4 and 6: up to 8% longer); streaming stores (plain
-// ones 31.9 and 45.4 us in the first line), plain loads (streaming ones 29.0
-// and 41.1: neighbouring waves share a line).
+// It is the slower by up to 5% for f32 rows of whole aligned groups of four around
+// 8M values (stochastic; 16776 x 500 14.6 -> 15.4).  Streaming stores (plain ones 31.9
+// and 45.4 us in the first line), plain loads (streaming ones 29.0 and 41.1:
+// neighbouring waves share a line).
 constexpr int kRowsUnroll = 3;
+// Groups of 16 bytes from which a thread takes three; us, one -> three, mean of ten
+// row lengths: f32 2M values 5.64 -> 5.78, 4M 8.96 -> 8.27, bf16 4M 6.62 -> 7.17, 8M
+// 10.4 -> 10.5, 16M 17.6 -> 16.5.
+constexpr int64_t kRowsManyGroups = (int64_t)3 << 18;
+// Values under which a lane takes one; us, 16 bytes -> one: f32 64K values 2.78 ->
+// 2.43, 128K 2.88 -> 2.56, 256K 2.97 -> 3.01, bf16 64K 2.97 -> 2.45, 128K 3.06 -> 2.55,
+// 256K 3.13 -> 2.99, 512K 3.26 -> 3.86 (the kernel before 3.3, 3.4, 3.5, 3.9).
+constexpr int64_t kRowsOneValue = (int64_t)1 << 18;
 // Workgroups along x: a grid dimension holds under 2^32 threads, which rows of 65
 // values reach at 139 GB; more go along y.
 constexpr int64_t kRowsGridX = (int64_t)1 << 22;
 
-template <int DT, int BS, bool STOCH>
+template <int DT, int BS, bool STOCH, int U, int VL>
 __global__ __launch_bounds__(kThreads) void fq_rows_kernel(const typename Elem<DT>::S* __restrict__ x,
                                                            typename Elem<DT>::S* __restrict__ y, int64_t groups,
                                                            int64_t cols, int64_t gp, const float* __restrict__ lut_g,
                                                            const uint8_t* __restrict__ band_g, uint64_t seed,
                                                            const uint64_t* __restrict__ seed_dev, uint64_t offset) {
     using E = Elem<DT>;
-    constexpr int V = E::V;
-    static_assert(BS % V == 0, "a group lies inside one block");
+    static_assert(VL == 1 || VL == E::V, "values per lane");
+    static_assert(BS % VL == 0, "a group lies inside one block");
     const uint64_t key = STOCH ? dither_key(seed + (seed_dev ? *seed_dev : 0ull)) : 0ull;
     __shared__ float lut_s[kLutSize];
     __shared__ uint32_t band_w[kBandSize / 4];
     const uint8_t* band_s = reinterpret_cast<const uint8_t*>(band_w);
     const int tid = threadIdx.x;
-    const int64_t l0 = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (kThreads * kRowsUnroll);
-    int64_t row[kRowsUnroll], col[kRowsUnroll];
-    u32x4 raw[kRowsUnroll];
+    const int64_t l0 = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (kThreads * U);
+    int64_t row[U], col[U];
+    RowsVec<DT, VL> raw[U];
     {
-        const int64_t r0 = l0 / gp;                    // uniform
-        int64_t r = r0, g = l0 - r0 * gp + tid;
+        // uniform; 64-bit divisions only where the tensor needs them
+        const int64_t r0 = (l0 >> 32) == 0 && (gp >> 32) == 0 ? (int64_t)((uint32_t)l0 / (uint32_t)gp) : l0 / gp;
+        int64_t r = r0, g = l0 - r0 * gp + tid, dr = 0;
         if (gp <= kThreads) {                          // 32-bit: g < gp + 256
             const uint32_t q = (uint32_t)g / (uint32_t)gp;
             r += q;
             g -= (int64_t)q * gp;
+            dr = (uint32_t)kThreads / (uint32_t)gp;
         } else if (g >= gp) {
             ++r;
             g -= gp;
         }
-        const int64_t dr = kThreads / gp, dg = kThreads - dr * gp;
+        const int64_t dg = kThreads - dr * gp;
 #pragma unroll
-        for (int u = 0; u < kRowsUnroll; ++u) {
+        for (int u = 0; u < U; ++u) {
             const bool live = l0 + u * kThreads + tid < groups;
             row[u] = live ? r : 0;
-            col[u] = live ? g * V : cols;              // past the row: zeros, nothing stored
-            // inside the row whatever the group (cols >= V)
-            const int64_t c = col[u] + V <= cols ? col[u] : cols - V;
-            raw[u] = *reinterpret_cast<const UnalignedVec<DT>*>(x + row[u] * cols + c);
+            col[u] = live ? g * VL : cols;             // past the row: zeros, nothing stored
+            // inside the row whatever the group (cols >= VL)
+            const int64_t c = col[u] + VL <= cols ? col[u] : cols - VL;
+            raw[u] = *reinterpret_cast<const RowsVec<DT, VL>*>(x + row[u] * cols + c);
             r += dr;
             g += dg;
             if (g >= gp) {
@@ -297,42 +315,66 @@ __global__ __launch_bounds__(kThreads) void fq_rows_kernel(const typename Elem<D
         }
     }
     stage_tables(lut_s, band_w, lut_g, band_g);
+    const int rest = (int)(cols & (VL - 1));           // uniform: values of a row's cut group
 #pragma unroll
-    for (int u = 0; u < kRowsUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
         const int64_t base = row[u] * cols + col[u];
-        float f[V];
-        E::unpack(raw[u], f);
-        const bool cut = col[u] + V > cols;
-        if (__builtin_amdgcn_ballot_w64(cut) != 0) {   // wave-uniform: a row ends in this wave
+        float f[VL];
+        if constexpr (VL == 1) {
+            f[0] = E::to_f(raw[u]);
+        } else {
+            E::unpack(raw[u], f);
+        }
+        const bool cut = col[u] + VL > cols;
+        if (__builtin_amdgcn_ballot_w64(cut) == 0) {   // wave-uniform: no row ends in this wave
+        } else if (rest == 0) {
+#pragma unroll
+            for (int e = 0; e < VL; ++e) f[e] = cut ? 0.0f : f[e];
+        } else if (VL == 8 && rest == 4) {
+            const bool some = col[u] < cols;
+#pragma unroll
+            for (int e = 0; e < VL / 2; ++e) {
+                f[e] = cut ? (some ? f[e + VL / 2] : 0.0f) : f[e];
+                f[e + VL / 2] = cut ? 0.0f : f[e + VL / 2];
+            }
+        } else {
             const int keep = (int)(cols - col[u] > 0 ? cols - col[u] : 0);   // values of a cut group
-            float g[V];
+            float g[VL];
 #pragma unroll
-            for (int e = 0; e < V; ++e) {
+            for (int e = 0; e < VL; ++e) {
                 g[e] = 0.0f;
-                // value e is loaded value V - keep + e
+                // value e is loaded value VL - keep + e
 #pragma unroll
-                for (int k = e + 1; k < V; ++k) g[e] = keep == V - (k - e) && k < V ? f[k] : g[e];
+                for (int k = e + 1; k < VL; ++k) g[e] = keep == VL - (k - e) ? f[k] : g[e];
             }
 #pragma unroll
-            for (int e = 0; e < V; ++e) f[e] = cut ? g[e] : f[e];
+            for (int e = 0; e < VL; ++e) f[e] = cut ? g[e] : f[e];
         }
         uint32_t m = 0;
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
+        for (int e = 0; e < VL; ++e) {
             const uint32_t a = __float_as_uint(f[e]) & 0x7fffffffu;
             m = m > a ? m : a;
         }
-        const FqScale s = fq_scale(group_umax<BS / V>(m), band_s);
-        float d[V];
+        if constexpr (VL == 1) m = lanes_umax<BS>(m);
+        else m = group_umax<BS / VL>(m);
+        const FqScale s = fq_scale(m, band_s);
+        float d[VL];
         const DitherVec dv = dither_vec(key, offset + (uint64_t)base);
 #pragma unroll
-        for (int e = 0; e < V; ++e) d[e] = STOCH ? dither_step(dv, e) : 0.0f;
-        fq_vector<V>(f, s, lut_s, STOCH, d);
+        for (int e = 0; e < VL; ++e) d[e] = STOCH ? dither_step(dv, e) : 0.0f;
+        fq_vector<VL>(f, s, lut_s, STOCH, d);
         if (!cut) {
-            st_stream((UnalignedVec<DT>)E::pack(f), reinterpret_cast<UnalignedVec<DT>*>(y + base));
-        } else {
+            if constexpr (VL == 1) y[base] = E::from_f(f[0]);
+            else st_stream((RowsVec<DT, VL>)E::pack(f), reinterpret_cast<RowsVec<DT, VL>*>(y + base));
+        } else if (VL == 8 && rest == 4) {
+            if constexpr (VL == 8) {
+                const u32x4 w = E::pack(f);
+                if (col[u] < cols) st_stream((u32x2_at2)u32x2_vec{w.x, w.y}, reinterpret_cast<u32x2_at2*>(y + base));
+            }
+        } else if (rest != 0) {
 #pragma unroll
-            for (int e = 0; e < V; ++e)
+            for (int e = 0; e < VL; ++e)
                 if (col[u] + e < cols) y[base + e] = E::from_f(f[e]);
         }
     }
@@ -965,16 +1007,25 @@ void launch_fq_typed(const void* x, void* y, int64_t rows, int64_t cols, bool st
     const int esize = (int)sizeof(S);
     const bool four = cols % 4 == 0 && (uintptr_t)x % (4 * esize) == 0 && (uintptr_t)y % (4 * esize) == 0;
     if (cols >= 4 * kRowsMinCols || (cols >= kRowsMinCols && !four)) {
-        const int64_t gp = (cols + BS - 1) / BS * (BS / V), groups = rows * gp;
-        const int64_t need = (groups + kThreads * kRowsUnroll - 1) / (kThreads * kRowsUnroll);
-        const dim3 grid((unsigned)(need < kRowsGridX ? need : kRowsGridX),
-                        (unsigned)((need + kRowsGridX - 1) / kRowsGridX));
-        if (stochastic)
-            fq_rows_kernel<DT, BS, true><<<grid, kThreads, 0, st>>>((const S*)x, (S*)y, groups, cols, gp, t.lut, t.band, seed,
-                                                                    seed_dev, offset);
+        auto run = [&](auto u, auto vl) {
+            constexpr int U = decltype(u)::value, VL = decltype(vl)::value;
+            const int64_t gp = (cols + BS - 1) / BS * (BS / VL), groups = rows * gp;
+            const int64_t need = (groups + kThreads * U - 1) / (kThreads * U);
+            const dim3 grid((unsigned)(need < kRowsGridX ? need : kRowsGridX),
+                            (unsigned)((need + kRowsGridX - 1) / kRowsGridX));
+            if (stochastic)
+                fq_rows_kernel<DT, BS, true, U, VL><<<grid, kThreads, 0, st>>>(
+                    (const S*)x, (S*)y, groups, cols, gp, t.lut, t.band, seed, seed_dev, offset);
+            else
+                fq_rows_kernel<DT, BS, false, U, VL><<<grid, kThreads, 0, st>>>(
+                    (const S*)x, (S*)y, groups, cols, gp, t.lut, t.band, seed, seed_dev, offset);
+        };
+        if (rows * cols < kRowsOneValue)
+            run(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
+        else if (rows * ((cols + V - 1) / V) < kRowsManyGroups)
+            run(std::integral_constant<int, 1>(), std::integral_constant<int, V>());
         else
-            fq_rows_kernel<DT, BS, false><<<grid, kThreads, 0, st>>>((const S*)x, (S*)y, groups, cols, gp, t.lut, t.band,
-                                                                     seed, seed_dev, offset);
+            run(std::integral_constant<int, kRowsUnroll>(), std::integral_constant<int, V>());
     } else {
         // short rows: 1..63 values one per lane, or whole 4-value groups under
         // 256 values (aligned) four per lane; R = 64 * VL / cols rows per wave

@@ -49,6 +49,31 @@ def test_fq_ragged_rows(cols, dt):
         assert torch.equal(_bits(got), _bits(_want(x, bs, u))), (rows, bs)
 
 
+# the tensors' sizes at which a lane takes 16 bytes instead of one value, and a
+# thread three groups instead of one: on both sides, with every cut group
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("cols", [65, 66, 67, 68, 69, 70, 71, 76, 1017, 4095])
+def test_fq_ragged_rows_sizes(cols, dt):
+    from axs.unified.hip_kernels import hip_fused_fake_quantize
+
+    per = 4 if dt == torch.float32 else 8
+    many = -(-(3 << 18) // -(-cols // per))
+    one = -(-(1 << 18) // cols)
+    g = torch.Generator().manual_seed(cols)
+    for rows in (one - 1, one, many - 1, many):
+        x = torch.randn(rows, cols, generator=g).to(dt)
+        x[rows // 2] *= 0.01
+        x[-1, -5:] = 0.0
+        buf = torch.empty(rows * cols + 1, dtype=dt, device=DEV)
+        xd = buf[1:].view(rows, cols).copy_(x)
+        got = hip_fused_fake_quantize(xd, 32).cpu()
+        assert torch.equal(_bits(got), _bits(_want(x, 32))), rows
+        if rows in (one, many):
+            u = oracle.uniform(SEED, 0, x.numel())
+            got = hip_fused_fake_quantize(x.to(DEV), 16, "stochastic", seed=SEED).cpu()
+            assert torch.equal(_bits(got), _bits(_want(x, 16, u))), rows
+
+
 def test_fq_ragged_rows_past_one_grid_dimension():
     """More groups than the threads of one grid dimension (2^32, three groups a
     thread): 140 GB of rows of 65 values, in place; rows around the border of a
