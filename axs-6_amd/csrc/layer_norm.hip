@@ -229,6 +229,9 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_vec_kernel(LnArgs a) {
 // and written.  Forward + backward, us, without -> with: 8192 x 4096 bf16 86.3
 // -> 76.3, 4096 x 8192 bf16 93.0 -> 82.2, 4096 x 8192 f32 128.7 -> 123.1; shorter
 // f32 rows have enough workgroups in flight and lose (8192 x 4096 119.8 -> 123).
+// AHEAD: a row's loads all go out first, past the row clamped, not under the row's
+// bound one vector after the other: 4096 x 4096 f32 79.9 -> 77.6; with fewer vectors
+// it loses (4096 x 3072 60.2 -> 64.9, 1024 x 2048 29.8 -> 30.6).
 template <int DT, int NT, int NV, bool STREAM, bool RAG>
 __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     using E = Elem<DT>;
@@ -247,10 +250,11 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     }
     const float inv_n = 1.0f / (float)a.cols;
     const size_t es = sizeof(typename E::S);
-    constexpr bool PF = DT != AXS6_F32 || NV >= 6;
+    constexpr bool PF = DT != AXS6_F32 || NV >= 6, AHEAD = PF || (NT == 256 && NV == 4);
     u32x4 nx[NV], nd[NV];
     float nmean = 0.0f, nrstd = 0.0f;
     // a row past the last reads the last; columns past the row read its last vector
+    // (AHEAD) or nothing
     auto fetch = [&](int64_t row) {
         const int64_t r = row < a.rows ? row : a.rows - 1;
         const char* xr = reinterpret_cast<const char*>(a.x) + r * a.cols * (int64_t)es;
@@ -258,8 +262,16 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int64_t vi = t + (int64_t)j * NT, at = vec_at<V, RAG>(vi < nvec ? vi : nvec - 1, a.cols);
-            nx[j] = load_raw<DT, STREAM, RAG>(xr, at);
-            nd[j] = load_raw<DT, STREAM, RAG>(dyr, at);
+            if constexpr (AHEAD) {
+                nx[j] = load_raw<DT, STREAM, RAG>(xr, at);
+                nd[j] = load_raw<DT, STREAM, RAG>(dyr, at);
+            } else {
+                nx[j] = nd[j] = u32x4{0u, 0u, 0u, 0u};
+                if (vi < nvec) {
+                    nx[j] = load_raw<DT, STREAM, RAG>(xr, at);
+                    nd[j] = load_raw<DT, STREAM, RAG>(dyr, at);
+                }
+            }
         }
         nmean = a.mean[r];
         nrstd = a.rstd[r];
@@ -284,7 +296,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
             E::unpack(cx[j], xv);
             E::unpack(cd[j], dv);
 #pragma unroll
-            for (int e = 0; e < V; ++e) dv[e] = vi < nvec ? dv[e] : 0.0f;
+            for (int e = 0; e < V; ++e) dv[e] = !AHEAD || vi < nvec ? dv[e] : 0.0f;
             const bool in = vi < nvec;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
