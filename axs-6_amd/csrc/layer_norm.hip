@@ -15,10 +15,10 @@
 // the backward; four rows per workgroup), else one 256-thread workgroup per
 // row -- so the statistics take one HBM read.  Rows that are not whole vectors,
 // and unaligned tensors, take the same form with unaligned 16-byte accesses
-// (RAG); a ragged row's last vector overlaps the one before.  Against the
-// generic form, which reads a value per lane and each row two or three times,
-// forward + backward, us: 8192 x 1001 bf16 64 -> 33, 8192 x 999 f32 60 -> 38,
-// 2048 x 4095 f32 64 -> 48 (whole vectors: 8192 x 1000 bf16 30).
+// (RAG; the backward from ragged_bwd_rows rows); a ragged row's last vector overlaps
+// the one before.  Against the generic form, which reads a value per lane and each
+// row two or three times, forward + backward, us: 8192 x 1001 bf16 64 -> 33, 8192 x
+// 999 f32 60 -> 38, 2048 x 4095 f32 64 -> 48 (whole vectors: 8192 x 1000 bf16 30).
 // The backward reads x and dy once per row: each thread keeps its columns'
 // dgamma/dbeta sums over the rows of its workgroup, the workgroup writes them
 // as one partial row (dgamma rows, then dbeta rows, one per workgroup), and a
@@ -597,6 +597,14 @@ int bwd_dispatch(const LnArgs& a, const LnShape& s, int64_t chunks, hipStream_t 
     return AXS6_OK;
 }
 
+// Rows from which the backward of ragged rows takes the vector form.  A workgroup
+// walks 16 rows, so few rows leave CUs idle, where the generic form has a workgroup
+// per row.  Backward, us, generic / vector: f32 32 x 2049 10.6 / 21.4, 1024 x 2049
+// 19.4 / 26.6, 2048 x 3001 31.7 / 29.4, 2048 x 8191 86 / 56; bf16 1024 x 4095 30.5 / 36.0,
+// 2048 x 8191 71.9 / 66.8; rows of a wave f32 256 x 1001 9.5 / 11.5, 512 x 1001 14.1 /
+// 12.8, 1024 x 515 14.2 / 11.2; of one vector a lane the vector form throughout.
+int64_t ragged_bwd_rows(const LnShape& s) { return s.nt == 256 ? 2048 : s.nv > 1 ? 512 : 0; }
+
 // Workgroups of the backward (= partial rows): about 16 rows each, at most 2048.
 int64_t bwd_chunks(int64_t rows) {
     if (rows <= 0) return 0;
@@ -631,6 +639,10 @@ extern "C" int axs6_layer_norm_forward(const void* x, int32_t dtype, int64_t row
     for (const void* p : ptrs)
         if (p && (uintptr_t)p % es != 0) return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: pointer not element-aligned", fn);
     LnShape s = ln_shape(dtype, cols, ptrs, 4, false);
+    // few ragged f32 rows of three or four vectors a lane: a workgroup per row is as
+    // fast (256 x 1001 4.3 against 4.5 us, 512 x 1001 4.6 both) and leaves x in the L2
+    // of the XCD whose backward reads it (261 x 1001 with the backward 14.0 against 15.4)
+    if (s.ragged && dtype == AXS6_F32 && s.nt == 64 && s.nv >= 3 && rows < 512) s.vec = false;
     LnArgs a{x, nullptr, gamma, beta, y, nullptr, mean, rstd, nullptr, rows, cols, eps};
     hipStream_t st = (hipStream_t)stream;
     if (dtype == AXS6_F32) rc = fwd_dispatch<AXS6_F32>(a, s, st);
@@ -669,6 +681,7 @@ extern "C" int axs6_layer_norm_backward(const void* dy, const void* x, int32_t d
             if (p && (uintptr_t)p % es != 0)
                 return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: pointer not element-aligned", fn);
         LnShape s = ln_shape(dtype, cols, ptrs, 4, true);
+        if (s.ragged && rows < ragged_bwd_rows(s)) s.vec = false;
         LnArgs a{x, dy, gamma, nullptr, nullptr, dx, const_cast<float*>(mean), const_cast<float*>(rstd),
                  reinterpret_cast<float*>(workspace), rows, cols, 0.0f};
         if (dtype == AXS6_F32) rc = bwd_dispatch<AXS6_F32>(a, s, chunks, st);

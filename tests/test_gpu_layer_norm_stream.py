@@ -30,7 +30,17 @@ CASES = [
     (262145, 264, torch.float16),
     (16400, 4097, torch.bfloat16),   # streamed, ragged
     (65600, 515, torch.float32),     # streamed, ragged, a wave per row
-    # the same forms below that size
+    # ragged rows on both sides of the row counts from which the backward takes the vector form
+    (511, 1001, torch.float32),
+    (512, 1001, torch.float32),
+    (513, 257, torch.float32),
+    (2047, 1027, torch.float32),
+    (2048, 1027, torch.float32),
+    (2048, 8191, torch.float32),
+    (2050, 2047, torch.float16),
+    (2048, 8191, torch.bfloat16),
+    (530, 515, torch.bfloat16),
+    # the streamed forms below their size
     (8192, 1024, torch.float32),
     (8191, 1024, torch.float32),
     (32771, 260, torch.float32),     # a wave per row, last group of one vector
