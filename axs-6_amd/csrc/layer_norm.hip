@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_vec_kernel(LnArgs a) {
     }
     const float inv_n = 1.0f / (float)a.cols;
     const size_t es = sizeof(typename E::S);
-    constexpr bool PF = DT != AXS6_F32 || NV >= 6, AHEAD = PF || (NT == 256 && NV == 4);
+    constexpr bool PF = DT != AXS6_F32 || NV >= 6, AHEAD = PF || NV == 4;
     u32x4 nx[NV], nd[NV];
     float nmean = 0.0f, nrstd = 0.0f;
     // a row past the last reads the last; columns past the row read its last vector
@@ -597,13 +597,17 @@ int bwd_dispatch(const LnArgs& a, const LnShape& s, int64_t chunks, hipStream_t 
     return AXS6_OK;
 }
 
-// Rows from which the backward of ragged rows takes the vector form.  A workgroup
-// walks 16 rows, so few rows leave CUs idle, where the generic form has a workgroup
-// per row.  Backward, us, generic / vector: f32 32 x 2049 10.6 / 21.4, 1024 x 2049
-// 19.4 / 26.6, 2048 x 3001 31.7 / 29.4, 2048 x 8191 86 / 56; bf16 1024 x 4095 30.5 / 36.0,
+// Rows from which the backward of ragged rows takes the vector form (up to four it
+// does too).  A workgroup walks 16 rows, so few rows leave CUs idle, where the generic
+// form has a workgroup per row.  Backward, us, generic / vector: f32 32 x 2049 10.6 / 21.4, 1024 x 2049
+// 19.4 / 26.6, 2048 x 3001 31.7 / 29.4, 1024 x 4095 27.4 / 29.8, 1365 x 6145 3 us the
+// slower, 2048 x 8191 86 / 56; bf16 1024 x 4095 30.5 / 36.0,
 // 2048 x 8191 71.9 / 66.8; rows of a wave f32 256 x 1001 9.5 / 11.5, 512 x 1001 14.1 /
 // 12.8, 1024 x 515 14.2 / 11.2; of one vector a lane the vector form throughout.
-int64_t ragged_bwd_rows(const LnShape& s) { return s.nt == 256 ? 2048 : s.nv > 1 ? 512 : 0; }
+int64_t ragged_bwd_rows(const LnShape& s, int dtype) {
+    if (s.nt == 256) return dtype == AXS6_F32 && s.nv >= 4 ? 1280 : 2048;
+    return s.nv > 1 ? 512 : 0;
+}
 
 // Workgroups of the backward (= partial rows): about 16 rows each, at most 2048.
 int64_t bwd_chunks(int64_t rows) {
@@ -681,7 +685,7 @@ extern "C" int axs6_layer_norm_backward(const void* dy, const void* x, int32_t d
             if (p && (uintptr_t)p % es != 0)
                 return fail(AXS6_ERR_INVALID_ARGUMENT, "%s: pointer not element-aligned", fn);
         LnShape s = ln_shape(dtype, cols, ptrs, 4, true);
-        if (s.ragged && rows < ragged_bwd_rows(s)) s.vec = false;
+        if (s.ragged && rows > 4 && rows < ragged_bwd_rows(s, dtype)) s.vec = false;
         LnArgs a{x, dy, gamma, nullptr, nullptr, dx, const_cast<float*>(mean), const_cast<float*>(rstd),
                  reinterpret_cast<float*>(workspace), rows, cols, 0.0f};
         if (dtype == AXS6_F32) rc = bwd_dispatch<AXS6_F32>(a, s, chunks, st);
