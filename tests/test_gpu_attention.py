@@ -272,3 +272,22 @@ def test_linear_group_matches_separate_without_gradients(m, K, sizes, dt, bias):
     assert all(torch.equal(y, s) for y, s in zip(ys, sep))
     ys[1].sum().backward()
     assert ws[1].grad is not None
+
+
+@pytest.mark.parametrize("dim,rows", [(1280, 64), (2048, 40), (512, 1)])
+def test_self_attention_groups_projections_without_gradients(dim, rows):
+    """The same in inference, at sizes whose projections take an inference form
+    stacked, alone or both: a hook on one of them changes no bit."""
+    import axs.unified as u
+
+    torch.manual_seed(5)
+    mha = u.AXSMultiheadAttentionUnified(dim, 8).to(DEV).eval()
+    x = torch.randn(1, rows, dim, generator=torch.Generator().manual_seed(6)).to(DEV)
+    with torch.no_grad():
+        torch.manual_seed(7)      # the probabilities' stochastic rounding
+        grouped = mha(x, x, x)
+        h = mha.q_proj.register_forward_hook(lambda m, i, o: None)
+        torch.manual_seed(7)
+        separate = mha(x, x, x)
+        h.remove()
+    assert torch.equal(grouped, separate)
