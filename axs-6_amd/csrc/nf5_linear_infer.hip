@@ -377,7 +377,7 @@ struct InferTile {
 // Adds the K splits' partial tiles in order (InferTile::store's layout) and
 // finishes them.  A workgroup takes 16 rows x 64 columns of a tile, a wave four
 // of the rows, so that its stores cover whole rows of 64.
-template <int BM, int MW, int NW>
+template <bool SCALED, int BM, int MW, int NW>
 __global__ __launch_bounds__(256) void infer_reduce_kernel(InferK k) {
     constexpr int TM = BM / (16 * MW), TN = kIN / (16 * NW), PARTS = BM / 16 * 2;
     const int part = (int)blockIdx.x % PARTS, tile = (int)blockIdx.x / PARTS;
@@ -390,16 +390,17 @@ __global__ __launch_bounds__(256) void infer_reduce_kernel(InferK k) {
     const float* p = k.partial + (int64_t)tile * (BM * kIN) +
                      ((wave * TN + jb % TN) * TM + ib % TM) * 256 + (cq * 16 + r) * 4;
     const int64_t stride = (int64_t)k.tiles_n * (BM * kIN);
-    const int sx = k.sx ? k.sx[row] + kScaleDown : 0;
+    const int sx = SCALED ? k.sx[row] + kScaleDown : 0;
     int sh[4] = {sx, sx, sx, sx};
     int again = 0;
-    f32x4m v = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4m v = *reinterpret_cast<const f32x4m*>(p);
+    if constexpr (SCALED) again = k.again[tile];
 #pragma unroll 4
-    for (int z = 0; z < k.splits; ++z) {
+    for (int z = 1; z < k.splits; ++z) {
         v += *reinterpret_cast<const f32x4m*>(p + z * stride);
-        if (k.again) again |= k.again[z * k.tiles_n + tile];
+        if constexpr (SCALED) again |= k.again[z * k.tiles_n + tile];
     }
-    if (again != 0) {
+    if (SCALED && again != 0) {
         // parts with exponents of their own: summed relative to the largest of
         // those of parts that are not 0
         int ref[4], top[4] = {INT_MIN, INT_MIN, INT_MIN, INT_MIN};
@@ -646,7 +647,7 @@ int run_infer(const InferK& k, hipStream_t st) {
         attr_set = true;
     }
     infer_gemm_kernel<DT, BM, MW, NW><<<(unsigned)(k.tiles_n * k.splits), kIThreads, lds, st>>>(k);
-    if (k.splits > 1) infer_reduce_kernel<BM, MW, NW><<<(unsigned)(k.tiles_n * (BM / 8)), 256, 0, st>>>(k);
+    if (k.splits > 1) infer_reduce_kernel<DT == AXS6_F32, BM, MW, NW><<<(unsigned)(k.tiles_n * (BM / 8)), 256, 0, st>>>(k);
     return check_launch("infer_gemm");
 }
 
